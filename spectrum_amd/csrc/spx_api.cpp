@@ -185,6 +185,7 @@ struct spx_sim {
    bool running = false;
    uint64_t run_first = 0, run_n = 0;
    bool keep_records = false;
+   uint64_t run_done = 0;              // trajectories finished when the control block was last read
    // SimulationMaster's tasks (src/simulation.hh:196-237): trajectory count, batch size, per-worker
    // maximum, the base name of the distribution files, the distributions to restore at the start
    int64_t task_n = 0, task_batch = 0, task_max_per_worker = 0;
@@ -869,9 +870,10 @@ int spx_begin(spx_sim* s, uint64_t first, uint64_t n_traj, const spx_rng* rng, i
    const int qi = P.alloc_index();
    if (qi < 0) return fail(s, SPX_ERR_STATE, "query table full");
    HIPCHK(s, P.set_query(qi, s->q.desc));
-   HIPCHK(s, P.push_queue(qi));
+   HIPCHK(s, P.push_queue(qi, n_traj));
    s->run_first = first;
    s->run_n = n_traj;
+   s->run_done = 0;
    s->running = true;
    return SPX_OK;
 }
@@ -880,6 +882,7 @@ static int read_stats(spx_sim* s, spx_run_stats* st, double wall, double kms, in
 {
    RunCtl ctl;
    HIPCHK(s, s->q.read_ctl(ctl, s->pool.stream));
+   s->run_done = ctl.done;
    if (st) {
       std::memset(st, 0, sizeof(*st));
       st->n_traj = s->run_n;
@@ -909,7 +912,7 @@ int spx_advance(spx_sim* s, int n_launches, spx_run_stats* st)
    auto w0 = std::chrono::steady_clock::now();
    s->pool.step_ms = s->pool.service_ms = 0.0;
    float ms = 0.f;
-   HIPCHK(s, s->pool.launch(n_launches, &ms));
+   HIPCHK(s, s->pool.launch(n_launches, s->run_n - std::min(s->run_done, s->run_n), &ms));
    double wall = std::chrono::duration<double>(std::chrono::steady_clock::now() - w0).count();
    return read_stats(s, st, wall, ms, n_launches);
 }
@@ -933,7 +936,7 @@ int spx_finish(spx_sim* s, spx_traj_record* records, spx_run_stats* st)
       if (ctl.done >= s->run_n) break;
       if (launches > guard) return fail(s, SPX_ERR_STATE, "run did not drain");
       float ms = 0.f;
-      HIPCHK(s, s->pool.launch(batch, &ms));
+      HIPCHK(s, s->pool.launch(batch, s->run_n - ctl.done, &ms));
       kms += ms;
       launches += batch;
       if (batch < 8) batch *= 2;
@@ -1405,7 +1408,7 @@ int spx_main_loop(spx_sim* s, const spx_rng* rng, spx_run_stats* st)
          if (done >= n_total) break;
          if (launches > guard) return fail(s, SPX_ERR_STATE, "run did not drain");
          float ms = 0.f;
-         HIPCHK(s, s->pool.launch(burst, &ms));
+         HIPCHK(s, s->pool.launch(burst, (uint64_t)(n_total - done), &ms));
          integ_ms += ms;
          launches += burst;
          if (burst < 8) burst *= 2;
@@ -1569,7 +1572,7 @@ static void server_loop(spx_server* S)
       for (SQuery* q : admitted) {
          hipError_t e = q->res.create(q->plan, q->hist_bins, q->first, q->n_traj, &q->rng, false, nullptr, nullptr, nullptr, q->pool->stream);
          if (e == hipSuccess) e = q->pool->set_query(q->qidx, q->res.desc);
-         if (e == hipSuccess) e = q->pool->push_queue(q->qidx);
+         if (e == hipSuccess) e = q->pool->push_queue(q->qidx, q->n_traj);
          if (e != hipSuccess) { server_fail(S, std::string("admit: ") + hipGetErrorString(e)); goto out; }
       }
       // one round of launches on every pool that has admitted queries; pools run on their own streams
@@ -1578,7 +1581,10 @@ static void server_loop(spx_server* S)
          bool any = false;
          for (Pool* pl : S->pools) {
             if (pl->host_queue.empty()) continue;
-            hipError_t e = pl->enqueue(S->o.launches_per_poll);
+            uint64_t live = 0;
+            for (const SQuery* q : S->running)   // this thread alone changes the list and the counters
+               if (q->pool == pl) live += q->n_traj - std::min<uint64_t>(q->ctl.done, q->n_traj);
+            hipError_t e = pl->enqueue(S->o.launches_per_poll, live);
             if (e != hipSuccess) { server_fail(S, std::string("launch: ") + hipGetErrorString(e)); goto out; }
             any = true;
          }

@@ -35,7 +35,11 @@ __device__ __forceinline__ spx_rng_desc load_rng(QueryPtr Q)
 // Slot states
 enum { SLOT_IDLE = 0, SLOT_RUN = 1, SLOT_START = 2, SLOT_EVENT = 3, SLOT_DONE = 4, SLOT_DISCARD = 5 };
 
-constexpr int BLOCK = 256;
+// One wave per workgroup: no lane works with another wave's, and single waves spread over the SIMDs of every CU and
+// refill one at a time where a workgroup of four waits for the last.  With the launches bounded to the slots a run can
+// fill (Pool::span): 20000 FP64 shock trajectories 1554 -> 1355 ms, 30000 of kappa ~ T r^2 128 -> 112 ms, 100000 FP64
+// modulation 316 -> 301 ms, against workgroups of four waves.
+constexpr int BLOCK = 64;
 
 // ---------------------------------------------------------------------------------------------
 // Wave helpers (64 lanes)
@@ -63,6 +67,47 @@ __device__ __forceinline__ void atomic_max_pos(unsigned long long* a, double v)
 {
    if (v >= 0.0) atomicMax(a, (unsigned long long)__double_as_longlong(v));
 }
+
+// ---------------------------------------------------------------------------------------------
+// Quads: the few-wave step kernels (V = 1) give every trajectory four neighbouring lanes.  All four hold the same
+// state and take the same branches; they split a derivative stencil by axis and the generator by block, and
+// read each other's parts through DPP moves within the quad (no LDS, no wait).
+// ---------------------------------------------------------------------------------------------
+constexpr int QUAD = 4;
+template <int K> __device__ __forceinline__ int quad_get(int v) { return __builtin_amdgcn_mov_dpp(v, K * 0x55, 0xf, 0xf, true); }
+template <int K> __device__ __forceinline__ float quad_get(float v)
+{
+   return __builtin_bit_cast(float, quad_get<K>(__builtin_bit_cast(int, v)));
+}
+template <int K> __device__ __forceinline__ double quad_get(double v)
+{
+   const uint64_t b = __builtin_bit_cast(uint64_t, v);
+   const uint32_t lo = (uint32_t)quad_get<K>((int)(uint32_t)b), hi = (uint32_t)quad_get<K>((int)(uint32_t)(b >> 32));
+   return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+__device__ __forceinline__ bool quad_any(bool b)   // over the three axes
+{
+   const int v = b ? 1 : 0;
+   return (quad_get<0>(v) | quad_get<1>(v) | quad_get<2>(v)) != 0;
+}
+template <typename R> __device__ __forceinline__ void own_rounding1(R& v) { if constexpr (is_f32<R>()) asm("" : "+v"(v)); }
+template <typename R> __device__ __forceinline__ void own_rounding1(v3<R>& v)
+{
+   own_rounding1(v.x);
+   own_rounding1(v.y);
+   own_rounding1(v.z);
+}
+// A sum whose next term follows in the same basic block: the FP32 unit contracts across statements, and without
+// this it would fuse the multiply of the term already in the sum instead of the next one's, as the loop does.
+template <typename... T> __device__ __forceinline__ void own_rounding(T&... v) { (own_rounding1(v), ...); }
+__device__ __forceinline__ int quad_lane() { return (int)threadIdx.x & (QUAD - 1); }
+// The slot of a lane in a step kernel, and whether the lane writes for it.
+template <int V> __device__ __forceinline__ uint64_t slot_of()
+{
+   const uint64_t i = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
+   return V == 1 ? i / QUAD : i;
+}
+template <int V> __device__ __forceinline__ bool slot_writer() { return V != 1 || quad_lane() == 0; }
 
 // ---------------------------------------------------------------------------------------------
 // Random draws: counter streams (Philox4x32-10 + Box-Muller pairs) or replayed buffers
@@ -168,6 +213,80 @@ __device__ __forceinline__ void next_normals(const spx_rng_desc& rng, uint64_t f
    S.nn += N;
 }
 
+// The same stream for a quad: when a draw needs a block that is not there, each lane generates one of the next four
+// (FP64: eight normals, FP32: sixteen) into an LDS ring of two such windows, and every lane reads its draws from
+// the ring.  A window is four consecutive blocks from a multiple of four, so the ring place of a draw is its
+// number modulo the ring, and a launch resumes anywhere in a window by generating it again.
+template <typename R> constexpr uint32_t block_draws() { return is_f32<R>() ? 4u : 2u; }
+template <typename R>
+struct QuadStream {
+   uint64_t traj;
+   uint32_t nn;          // normal draws consumed
+   uint32_t end;         // blocks generated so far (a multiple of four)
+   bool exhausted;
+   R* ring;              // this quad's 2 * QUAD * block_draws places
+};
+template <typename R>
+__device__ __forceinline__ void next_window(const spx_rng_desc& rng, QuadStream<R>& S)
+{
+   constexpr uint32_t ND = block_draws<R>(), RING = 2 * QUAD * ND;
+   const uint32_t blk = S.end + (uint32_t)quad_lane();
+   R* w = S.ring + (blk * ND) % RING;
+   if constexpr (is_f32<R>()) {
+      float n0, n1, n2, n3;
+      normal_quad_f32(rng.seed, S.traj, blk, n0, n1, n2, n3);
+      w[0] = n0; w[1] = n1; w[2] = n2; w[3] = n3;
+   }
+   else {
+      double c, s;
+      normal_pair_f64(rng.seed, S.traj, blk, c, s);
+      w[0] = c; w[1] = s;
+   }
+   S.end += (uint32_t)QUAD;
+}
+// The window of the next draw; from here on a call needs at most one window more.
+template <typename R>
+__device__ __forceinline__ void prime_normals(const spx_rng_desc& rng, QuadStream<R>& S)
+{
+   S.end = (S.nn / block_draws<R>()) & ~(uint32_t)(QUAD - 1);
+   if (rng.mode != 1) next_window(rng, S);
+}
+template <typename R, int N>
+__device__ __forceinline__ void next_normals(const spx_rng_desc& rng, uint64_t first, QuadStream<R>& S, R (&out)[N])
+{
+   static_assert(N >= 1 && N <= 3, "one to three draws per call");
+   constexpr uint32_t ND = block_draws<R>(), RING = 2 * QUAD * ND;
+   if (rng.mode == 1) {
+      const uint64_t base = (S.traj - first) * (uint64_t)rng.normal_stride;
+#pragma unroll
+      for (int i = 0; i < N; i++) {
+         const uint32_t k = S.nn + (uint32_t)i;
+         if ((int64_t)k >= rng.normal_stride) { S.exhausted = true; out[i] = R(0); }
+         else out[i] = R(rng.normals[base + k]);
+      }
+      S.nn += N;
+      return;
+   }
+   if ((S.nn + (uint32_t)N - 1u) / ND >= S.end) next_window(rng, S);
+   // the lanes of a wave run in step and its LDS accesses stay in order: only the compiler must not move them
+   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+   __builtin_amdgcn_wave_barrier();
+   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+   for (int i = 0; i < N; i++) out[i] = S.ring[(S.nn + (uint32_t)i) % RING];
+   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+   __builtin_amdgcn_wave_barrier();
+   S.nn += N;
+}
+// The stream type of a step kernel's form, and its LDS.
+template <typename R, int V> struct StreamOf { typedef NormalStream<R> type; };
+template <typename R> struct StreamOf<R, 1> { typedef QuadStream<R> type; };
+template <typename R, int V> struct RingLDS { __device__ __forceinline__ void bind(NormalStream<R>&) {} };
+template <typename R> struct RingLDS<R, 1> {
+   R place[BLOCK / QUAD][2 * QUAD * block_draws<R>()];
+   __device__ __forceinline__ void bind(QuadStream<R>& S) { S.ring = place[threadIdx.x / QUAD]; }
+};
+
 __device__ __forceinline__ double next_uniform(const spx_rng_desc& rng, uint64_t first, uint64_t traj, uint32_t& nu, bool& exhausted)
 {
    const uint32_t k = nu++;
@@ -204,8 +323,8 @@ __device__ __forceinline__ void pos_sample(PlanPtr P, const spx_rng_desc& rng, u
 // ---------------------------------------------------------------------------------------------
 // |x - origin| of a sphere boundary in the step type (FP32 from the FP64 offset): the distance the sphere's
 // delta subtracts the radius from
-template <typename R>
-__device__ __forceinline__ R sphere_dist(const SPX_CP spx_bnd_desc& b, double x, double y, double z)
+template <typename R, typename BB>
+__device__ __forceinline__ R sphere_dist(BB& b, double x, double y, double z)
 {
    if constexpr (is_f32<R>()) {
       const v3<float> d = mk<float>((float)(x - b.origin[0]), (float)(y - b.origin[1]), (float)(z - b.origin[2]));
@@ -216,8 +335,8 @@ __device__ __forceinline__ R sphere_dist(const SPX_CP spx_bnd_desc& b, double x,
 
 // With R = float the distance to a sphere or plane is formed in FP32 from the FP64 offset (the FP32
 // step's crossing test); time and momentum boundaries and every normal stay in FP64.
-template <typename R = double>
-__device__ __forceinline__ double bnd_eval(const SPX_CP spx_bnd_desc& b, int cross_left, bool gc, double t, double x, double y, double z,
+template <typename R = double, typename BB>
+__device__ __forceinline__ double bnd_eval(BB& b, int cross_left, bool gc, double t, double x, double y, double z,
                                            double m0, double m1, double m2, double* nrm)
 {
    if constexpr (is_f32<R>()) {
@@ -466,8 +585,8 @@ struct ColdLDS {
 
 
 // TrajectoryBase::TimeBoundaryProximityCheck (src/trajectory_base.cc:151-179)
-template <int FWD, typename HOT>
-__device__ __forceinline__ double time_proximity(PlanPtr P, const HOT& H, double dt, double dmax)
+template <int FWD, typename PP, typename HOT>
+__device__ __forceinline__ double time_proximity(PP P, const HOT& H, double dt, double dmax)
 {
    typedef typename HOT::real R;
    double dn = FWD ? -divc_d<R>(sp_large * dmax, c_code) : divc_d<R>(sp_large * dmax, c_code);
@@ -499,9 +618,9 @@ __device__ __forceinline__ double time_proximity(PlanPtr P, const HOT& H, double
 // 2 = an event was queued.  HOT is the transport's register state: t, x, y, z, the boundary arrays
 // bd / bdo / bst and the momentum accessors m0() / m1() / m2() (Parker keeps (p, 0, 0), the guiding centre
 // (p_perp, 0, p_par), the field line (0, 0, p_par), the full orbit (px, py, pz)) and reflect_mom() (a reflecting wall reverses p_par of a guiding centre,
-// src/trajectory_guiding.hh:121-124).
-template <bool GC, typename HOT>
-__device__ __forceinline__ int handle_boundaries(PlanPtr P, LaunchPtr L, uint64_t slot,
+// src/trajectory_guiding.hh:121-124).  Pc is the plan in memory, for what only a crossing reads.
+template <bool GC, int V = 0, typename PP, typename HOT>
+__device__ __forceinline__ int handle_boundaries(PP P, PlanPtr Pc, LaunchPtr L, uint64_t slot,
                                                  HOT& H, ColdLDS& C, int tid)
 {
    typedef typename HOT::real R;
@@ -511,7 +630,7 @@ __device__ __forceinline__ int handle_boundaries(PlanPtr P, LaunchPtr L, uint64_
    for (int b = 0; b < SPX_MAX_BND; b++) {
       if (b < P->n_bnd) {
          // ComputeBoundary (src/boundary_base.cc:105-127); a slot's recurrent bit is its boundary's (status0)
-         const SPX_CP spx_bnd_desc& B = P->bnd[b];
+         const auto& B = P->bnd[b];
          double d;
          if (B.kind == SPX_BK_SPHERE) {
             if (!B.same_origin) sdist = sphere_dist<R>(B, H.x, H.y, H.z);
@@ -559,12 +678,14 @@ __device__ __forceinline__ int handle_boundaries(PlanPtr P, LaunchPtr L, uint64_
             if (H.bst[b] & SPX_BND_TERMINAL) out |= 1;
          }
       }
-      if (active >= 0 && bnd_has_action(P, active)) {
+      if (active >= 0 && bnd_has_action(Pc, active)) {
+         if (slot_writer<V>()) {
          ev_field(L, cls, EV_T, slot) = H.t; ev_field(L, cls, EV_X, slot) = H.x; ev_field(L, cls, EV_Y, slot) = H.y;
          ev_field(L, cls, EV_Z, slot) = H.z; ev_field(L, cls, EV_M0, slot) = H.m0(); ev_field(L, cls, EV_M1, slot) = H.m1();
          ev_field(L, cls, EV_M2, slot) = H.m2(); ev_field(L, cls, EV_AMP, slot) = C.amp[tid]; ev_field(L, cls, EV_WGT, slot) = C.wgt[tid];
          L->ev_bnd[cls * L->n_lanes + slot] = active;
          L->ev_pending[slot] |= (1 << cls);
+         }
          out |= 2;
       }
    }

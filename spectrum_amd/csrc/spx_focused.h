@@ -52,8 +52,8 @@ __device__ __forceinline__ void fc_contract(FcFields<R>& F, v3<R> U, v3<R> B, co
 // GetFields with the focused mask at a position for momentum magnitude pm; ds_prev is the smooth shock's
 // hidden coordinate (read for dmax, then set to this evaluation's).  Returns false on
 // ExFieldError (|B| below sp_tiny).
-template <typename R, int BG>
-__device__ __forceinline__ bool fc_fields(const SPX_CP spx_bg_t<R>& bg, double t, double x, double y, double z, R pm, R& ds_prev, FcFields<R>& F)
+template <typename R, int BG, typename BD>
+__device__ __forceinline__ bool fc_fields(BD& bg, double t, double x, double y, double z, R pm, R& ds_prev, FcFields<R>& F)
 {
    F.dmax = bg_dmax<R, BG>(bg, x, y, z, ds_prev);
    if constexpr (BG == SPX_BG_GRID) {
@@ -175,7 +175,7 @@ template <typename R, int BG>
 __device__ int fc_set_start(PlanPtr P, QueryPtr Q, LaunchPtr L, const spx_rng_desc& rng, uint64_t slot,
                             uint64_t traj, uint32_t& nu)
 {
-   const SPX_CP spx_bg_t<R>& bg = PlanView<R>::bg(P);
+   auto& bg = PlanView<R>::bg(P);
    const uint64_t first = Q->first;
    const double t = P->it_t;
    bool ex = false;
@@ -249,7 +249,7 @@ struct FcHot {
 template <typename R, int BG, int FWD>
 __device__ __forceinline__ int fc_step(PlanPtr P, LaunchPtr L, uint64_t slot, FcHot<R>& H, ColdLDS& C, int tid, int& bflags)
 {
-   const SPX_CP spx_bg_t<R>& bg = PlanView<R>::bg(P);
+   auto& bg = PlanView<R>::bg(P);
    const FcFields<R>& F = H.F;
    const R p = R(H.p), mu = R(H.mu);
    const R v = p * (VelP(p) / p);
@@ -275,7 +275,7 @@ __device__ __forceinline__ int fc_step(PlanPtr P, LaunchPtr L, uint64_t slot, Fc
       H.x -= (double)(dtv * drift.x); H.y -= (double)(dtv * drift.y); H.z -= (double)(dtv * drift.z);
       H.p -= (double)(dtv * slope_p); H.mu -= (double)(dtv * slope_mu);
    }
-   bflags = handle_boundaries<false>(P, L, slot, H, C, tid);
+   bflags = handle_boundaries<false>(P, P, L, slot, H, C, tid);
    if (!(bflags & 1)) {
       H.ds_dm = H.ds;
       if (!fc_fields<R, BG>(bg, H.t, H.x, H.y, H.z, R(H.p), H.ds, H.F)) return 1;

@@ -32,8 +32,8 @@ struct GcFields {
 // of transpose(fa) * G.  The smooth shock's derivatives are analytic (src/background_smooth_shock.cc:159-187)
 // and its dmax reads the shock coordinate of the previous evaluation, ds_prev (set to this one's); the
 // discontinuous shock has none (src/background_shock.cc:116-128).  Returns false on ExFieldError.
-template <typename R, int BG>
-__device__ __forceinline__ bool gc_fields(const SPX_CP spx_bg_t<R>& bg, double t, double x, double y, double z, R pm, R& ds_prev,
+template <typename R, int BG, int V = 0, typename BD>
+__device__ __forceinline__ bool gc_fields(BD& bg, double t, double x, double y, double z, R pm, R& ds_prev,
                                           GcFields<R>& F)
 {
    F.dmax = bg_dmax<R, BG>(bg, x, y, z, ds_prev);
@@ -92,10 +92,8 @@ __device__ __forceinline__ bool gc_fields(const SPX_CP spx_bg_t<R>& bg, double t
       v3<R> gbm = mk<R>(R(0), R(0), R(0));
       v3<R> dc = mk<R>(R(0), R(0), R(0));
       if constexpr (is_f32<R>()) dc = rel(bg, x, y, z);   // FP32 stencil points relative to the origin
-      // the frame vectors rotate through e (moves instead of a select of each component per point)
-      v3<R> e = fa[0], e_next = fa[1];
-#pragma unroll 1
-      for (int k = 0; k < 3; k++) {
+      // the derivative of B and |B| along e
+      auto along = [&](v3<R> e, v3<R>& gB, R& gm) {
          R dr = r_g;
          v3<R> Ud, Bf, Bb;
          R dsd;
@@ -112,9 +110,11 @@ __device__ __forceinline__ bool gc_fields(const SPX_CP spx_bg_t<R>& bg, double t
             bg_eval<R, BG>(bg, t, xf - (double)(dr * e.x), yf - (double)(dr * e.y), zf - (double)(dr * e.z), 2, Ud, Bb, dsd);
          }
          const R idr = is_f32<R>() ? R(0.5) / r_g : R(0);   // FP32: one reciprocal per point
-         const v3<R> gB = is_f32<R>() ? idr * (Bf - Bb) : (Bf - Bb) / dr;
-         const R gm = is_f32<R>() ? (norm(Bf) - norm(Bb)) * idr : (norm(Bf) - norm(Bb)) / dr;
-         if (k == 0) {
+         gB = is_f32<R>() ? idr * (Bf - Bb) : (Bf - Bb) / dr;
+         gm = is_f32<R>() ? (norm(Bf) - norm(Bb)) * idr : (norm(Bf) - norm(Bb)) / dr;
+      };
+      auto add = [&](bool first, v3<R> e, v3<R> gB, R gm) {
+         if (first) {
             g01 = e.x * gB.y; g02 = e.x * gB.z; g10 = e.y * gB.x; g12 = e.y * gB.z; g20 = e.z * gB.x; g21 = e.z * gB.y;
             gbm = mk<R>(e.x * gm, e.y * gm, e.z * gm);
          }
@@ -122,8 +122,28 @@ __device__ __forceinline__ bool gc_fields(const SPX_CP spx_bg_t<R>& bg, double t
             g01 += e.x * gB.y; g02 += e.x * gB.z; g10 += e.y * gB.x; g12 += e.y * gB.z; g20 += e.z * gB.x; g21 += e.z * gB.y;
             gbm.x += e.x * gm; gbm.y += e.y * gm; gbm.z += e.z * gm;
          }
-         e = e_next;
-         e_next = fa[2];
+      };
+      if constexpr (V == 1) {   // each lane of the quad takes one axis; the terms are added in the same order
+         const int q = quad_lane();
+         v3<R> gB;
+         R gm;
+         along(q == 0 ? fa[0] : (q == 1 ? fa[1] : fa[2]), gB, gm);
+         add(true, fa[0], mk<R>(quad_get<0>(gB.x), quad_get<0>(gB.y), quad_get<0>(gB.z)), quad_get<0>(gm));
+         add(false, fa[1], mk<R>(quad_get<1>(gB.x), quad_get<1>(gB.y), quad_get<1>(gB.z)), quad_get<1>(gm));
+         add(false, fa[2], mk<R>(quad_get<2>(gB.x), quad_get<2>(gB.y), quad_get<2>(gB.z)), quad_get<2>(gm));
+      }
+      else {
+         // the frame vectors rotate through e (moves instead of a select of each component per point)
+         v3<R> e = fa[0], e_next = fa[1];
+#pragma unroll 1
+         for (int k = 0; k < 3; k++) {
+            v3<R> gB;
+            R gm;
+            along(e, gB, gm);
+            add(k == 0, e, gB, gm);
+            e = e_next;
+            e_next = fa[2];
+         }
       }
       F.gradBmag = gbm;
       const v3<R> curlB = mk<R>(g12 - g21, g20 - g02, g01 - g10);
@@ -155,8 +175,8 @@ __device__ __forceinline__ R hyp_series_11(R c, R z)
    return sum;
 }
 
-template <typename R>
-__device__ __forceinline__ R hyp2f1_11(const SPX_CP spx_df_t<R>& df, R z)
+template <typename R, typename DD>
+__device__ __forceinline__ R hyp2f1_11(DD& df, R z)
 {
    if (z < R(0.5)) return hyp_series_11(df.hyp_c, z);
    const R w = R(1) - z;
@@ -166,8 +186,8 @@ __device__ __forceinline__ R hyp2f1_11(const SPX_CP spx_df_t<R>& df, R z)
 // DiffusionWNLTConstant::EvaluateDiffusion (src/diffusion_other.cc:215-245) over DiffusionQLTConstant's
 // component 2 (:145-149), with DiffusionWNLTRampVLISM's k_min and amplitudes at the position (:301-328):
 // kappa_perp into K0 and, when comp2, D_mumu into K2.
-template <typename R>
-__device__ __noinline__ void wnlt_k(const SPX_CP spx_df_t<R>& df, bool comp2, double x, double y, double z, R pmag, R mu, R Bmag, R& K0, R& K2)
+template <typename R, typename DD>
+__device__ __noinline__ void wnlt_k(DD& df, bool comp2, double x, double y, double z, R pmag, R mu, R Bmag, R& K0, R& K2)
 {
    R k_min = df.k_min, A2A = df.A2A, A2T = df.A2T, A2L = df.A2L;
    if (df.kind == SPX_DF_WNLT_RAMP) {
@@ -204,8 +224,8 @@ __device__ __noinline__ void wnlt_k(const SPX_CP spx_df_t<R>& df, bool comp2, do
 // Strauss / Potgieter models read (src/diffusion_other.cc:886-906, :968-988).
 // XD compiles in the models that depend on mu and position (WNLT) or on the region (Strauss / Potgieter,
 // SOQLT), kept out of the kernels of the other models.
-template <typename R, bool XD>
-__device__ __forceinline__ R gc_kperp(const SPX_CP spx_df_t<R>& df, R pmag, R mu, R Bmag, double x, double y, double z, bool outer)
+template <typename R, bool XD, typename DD>
+__device__ __forceinline__ R gc_kperp(DD& df, R pmag, R mu, R Bmag, double x, double y, double z, bool outer)
 {
    if constexpr (XD) {
       if (df.kind == SPX_DF_STRAUSS || df.kind == SPX_DF_POTGIETER) {
@@ -241,8 +261,8 @@ __device__ __forceinline__ R gc_kperp(const SPX_CP spx_df_t<R>& df, R pmag, R mu
 // and its mu derivative, analytic for the isotropic model (src/diffusion_other.cc:64-79) and the forward
 // difference of DiffusionBase::GetMuDerivative (src/diffusion_base.cc:226-255) for DiffusionQLTConstant
 // (src/diffusion_other.cc:145-149); the other models have no component 2.
-template <typename R, bool XD>
-__device__ __forceinline__ void gc_dmumu(const SPX_CP spx_df_t<R>& df, R pmag, R Bmag, R mu, double x, double y, double z, R& Dmumu, R& Vmu)
+template <typename R, bool XD, typename DD>
+__device__ __forceinline__ void gc_dmumu(DD& df, R pmag, R Bmag, R mu, double x, double y, double z, R& Dmumu, R& Vmu)
 {
    if (XD && (df.kind == SPX_DF_WNLT || df.kind == SPX_DF_WNLT_RAMP)) {
       R K0, K2;
@@ -272,8 +292,8 @@ __device__ __forceinline__ void gc_dmumu(const SPX_CP spx_df_t<R>& df, R pmag, R
 // TrajectoryGuidingDiff::DiffusionCoeff (src/trajectory_guiding_diff.cc:72-98): D_perp and the
 // drift V_perp = grad_perp D_perp in the field-aligned frame.  Only the rigidity power law has a
 // spatial derivative (src/diffusion_other.cc:818-823), and only through |B|.
-template <typename R, bool XD>
-__device__ __forceinline__ void gc_perp(const SPX_CP spx_df_t<R>& df, const GcFields<R>& F, const v3<R>* fa, R pmag, R mu,
+template <typename R, bool XD, typename DD>
+__device__ __forceinline__ void gc_perp(DD& df, const GcFields<R>& F, const v3<R>* fa, R pmag, R mu,
                                         double x, double y, double z, bool outer, R& Dperp, v3<R>& Vperp)
 {
    Dperp = gc_kperp<R, XD>(df, pmag, mu, F.Bmag, x, y, z, outer);
@@ -365,7 +385,7 @@ template <typename R, int BG>
 __device__ int gc_set_start(PlanPtr P, QueryPtr Q, LaunchPtr L, const spx_rng_desc& rng, uint64_t slot,
                             uint64_t traj, uint32_t& nu)
 {
-   const SPX_CP spx_bg_t<R>& bg = PlanView<R>::bg(P);
+   auto& bg = PlanView<R>::bg(P);
    const uint64_t first = Q->first;
    const double t = P->it_t;
    bool ex = false;
@@ -417,7 +437,7 @@ __global__ __launch_bounds__(BLOCK) void gc_service(const Launch* __restrict__ L
 }
 
 // ---- step kernel -----------------------------------------------------------------------------
-template <typename R>
+template <typename R, int V>
 struct GcHot {
    double t, x, y, z, pp, pl;                   // time, position, (p_perp, p_par)
    double pf;                                   // |p| of the last field evaluation
@@ -425,7 +445,7 @@ struct GcHot {
    R ds_prev;                                   // BackgroundSmoothShock's hidden coordinate (smooth shock only)
    double bd[SPX_MAX_BND], bdo[SPX_MAX_BND];
    int bst[SPX_MAX_BND];
-   NormalStream<R> rs;
+   typename StreamOf<R, V>::type rs;
    int32_t steps;
    typedef R real;
    __device__ __forceinline__ double m0() const { return pp; }
@@ -438,12 +458,12 @@ struct GcHot {
 // DiffusionCoeff, DriftCoeff, PhysicalStep (src/trajectory_guiding_diff.cc:324-332 then
 // src/trajectory_guiding_scatt.cc:255-262), EulerPitchAngleScatt (:81-106), Slopes, EulerPerpDiffSlopes
 // (src/trajectory_guiding_diff.cc:123-140), the Euler RKStep, boundaries and the end-of-step fields.
-template <typename R, int BG, bool XD>
-__device__ __forceinline__ int gc_step(PlanPtr P, LaunchPtr L, const spx_rng_desc& rng,
-                                       uint64_t first, uint64_t slot, GcHot<R>& H, ColdLDS& C, int tid, int& bflags)
+template <typename R, int BG, bool XD, int V, typename PP>
+__device__ __forceinline__ int gc_step(PP P, PlanPtr Pc, LaunchPtr L, const spx_rng_desc& rng,
+                                       uint64_t first, uint64_t slot, GcHot<R, V>& H, ColdLDS& C, int tid, int& bflags)
 {
-   const SPX_CP spx_bg_t<R>& bg = PlanView<R>::bg(P);
-   const SPX_CP spx_df_t<R>& df = PlanView<R>::df(P);
+   auto& bg = PlanView<R>::bg(P);
+   auto& df = PlanView<R>::df(P);
    // the four guiding-centre transports differ in two terms: pitch-angle scattering (GuidingScatt,
    // GuidingDiffScatt) and perpendicular diffusion (GuidingDiff, GuidingDiffScatt); without them the
    // step draws no numbers for them and its coefficients are zero
@@ -564,10 +584,10 @@ __device__ __forceinline__ int gc_step(PlanPtr P, LaunchPtr L, const spx_rng_des
       H.pl = pld + (double)(dtv * slope_pl);
       if (perp_step) { H.x += (double)dr.x; H.y += (double)dr.y; H.z += (double)dr.z; }
    }
-   bflags = handle_boundaries<true>(P, L, slot, H, C, tid);
+   bflags = handle_boundaries<true, V>(P, Pc, L, slot, H, C, tid);
    if (!(bflags & 1)) {
       H.pf = sqrt_d<R>(H.pp * H.pp + H.pl * H.pl);
-      if (!gc_fields<R, BG>(bg, H.t, H.x, H.y, H.z, R(H.pf), H.ds_prev, H.F)) return 1;
+      if (!gc_fields<R, BG, V>(bg, H.t, H.x, H.y, H.z, R(H.pf), H.ds_prev, H.F)) return 1;
    }
    H.steps++;
    if (H.steps > P->max_steps) return 4;
@@ -576,23 +596,20 @@ __device__ __forceinline__ int gc_step(PlanPtr P, LaunchPtr L, const spx_rng_des
    return 0;
 }
 
-// SPX_GC_WAVES resident waves per SIMD for the step kernel (0: the compiler's own register budget).
+// Resident waves per SIMD asked of the compiler for the V = 0 step kernel (1: its own register budget).
 #ifndef SPX_GC_WAVES
-#define SPX_GC_WAVES 0
-#endif
-#if SPX_GC_WAVES > 0
-#define SPX_GC_ATTR __attribute__((amdgpu_waves_per_eu(SPX_GC_WAVES)))
-#else
-#define SPX_GC_ATTR
+#define SPX_GC_WAVES 1
 #endif
 
-template <typename R, int BG, bool XD>
-__global__ __launch_bounds__(BLOCK) SPX_GC_ATTR void gc_step_kernel(const Launch* __restrict__ Lg)
+template <typename R, int BG, bool XD, int V>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(V == 1 ? 1 : SPX_GC_WAVES))) void gc_step_kernel(const Launch* __restrict__ Lg)
 {
    const LaunchPtr Lp = (LaunchPtr)Lg;
    __shared__ ColdLDS C;
    const int tid = threadIdx.x;
-   const uint64_t slot = (uint64_t)blockIdx.x * BLOCK + tid;
+   __shared__ RingLDS<R, V> ring;
+   const uint64_t slot = slot_of<V>();
+   const bool writer = slot_writer<V>();
    // the slots of a wave work for one query (the pool size is a multiple of the block size)
    const int q = __builtin_amdgcn_readfirstlane(Lp->slot_q[slot]);
    const bool run = q >= 0 && Lp->active[slot] == SLOT_RUN;
@@ -601,7 +618,7 @@ __global__ __launch_bounds__(BLOCK) SPX_GC_ATTR void gc_step_kernel(const Launch
    const PlanPtr P = plan_of(Q);
    const spx_rng_desc rng = load_rng(Q);
    const uint64_t first = Q->first;
-   GcHot<R> H;
+   GcHot<R, V> H;
    if (run) {
       const uint64_t n = Lp->n_lanes;
       H.t = Lp->t[slot]; H.x = Lp->x[slot]; H.y = Lp->y[slot]; H.z = Lp->z[slot]; H.pp = Lp->m0[slot]; H.pl = Lp->m2[slot];
@@ -612,6 +629,7 @@ __global__ __launch_bounds__(BLOCK) SPX_GC_ATTR void gc_step_kernel(const Launch
       H.pf = Lp->pf[slot];
       H.steps = (int32_t)Lp->steps[slot];
       H.rs.traj = Lp->traj[slot]; H.rs.nn = Lp->nn[slot]; H.rs.exhausted = false;
+      ring.bind(H.rs);
       prime_normals<R>(rng, H.rs);
       C.amp[tid] = Lp->amp[slot]; C.wgt[tid] = Lp->wgt[slot]; C.dt_adapt[tid] = Lp->dt_adapt[slot];
 #pragma unroll
@@ -629,7 +647,10 @@ __global__ __launch_bounds__(BLOCK) SPX_GC_ATTR void gc_step_kernel(const Launch
    int st = run ? SLOT_RUN : SLOT_IDLE;
    int exc = 0;
    unsigned long long steps_here = 0;
-   for (int it = 0; it < Lp->steps_per_launch; it++) {
+   HotPlan<R> hot;
+   if constexpr (V == 1 && !is_f32<R>()) load_hot(hot, P);
+   const int n_steps = Lp->steps_per_launch;
+   for (int it = 0; it < n_steps; it++) {
       if (__ballot(st == SLOT_RUN) == 0) break;
       if (st != SLOT_RUN) continue;
       PlanPtr Pi = P;
@@ -637,7 +658,12 @@ __global__ __launch_bounds__(BLOCK) SPX_GC_ATTR void gc_step_kernel(const Launch
       LaunchPtr Li = Lp;
       asm volatile("" : "+s"(Li));
       int bflags = 0;
-      const int e = gc_step<R, BG, XD>(Pi, Li, rng, first, slot, H, C, tid, bflags);
+      int e;
+      if constexpr (V == 1 && !is_f32<R>()) {
+         const HotPlan<R>* h = &hot;
+         e = gc_step<R, BG, XD, V>(h, Pi, Li, rng, first, slot, H, C, tid, bflags);
+      }
+      else e = gc_step<R, BG, XD, V>(Pi, Pi, Li, rng, first, slot, H, C, tid, bflags);
       steps_here++;
       if (e != 0) { exc = e; st = SLOT_DISCARD; }
       else if (bflags & 1) st = SLOT_DONE;
@@ -645,10 +671,10 @@ __global__ __launch_bounds__(BLOCK) SPX_GC_ATTR void gc_step_kernel(const Launch
    }
    LaunchPtr Ls = Lp;
    asm volatile("" : "+s"(Ls));
-   unsigned long long s = steps_here;
+   unsigned long long s = writer ? steps_here : 0;
    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
    if (lane_id() == 0 && s) atomicAdd(&Q->ctl->steps_executed, s);
-   if (!run) return;
+   if (!run || !writer) return;
    const uint64_t n = Ls->n_lanes;
    Ls->active[slot] = st;
    Ls->ex_code[slot] = exc;
@@ -669,20 +695,24 @@ __global__ __launch_bounds__(BLOCK) SPX_GC_ATTR void gc_step_kernel(const Launch
    }
 }
 
-template <typename R, int BG, bool XD>
+template <typename R, int BG, bool XD, int M>
 static hipError_t launch_gc_bg(uint64_t n_lanes, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
 {
-   const unsigned grid = (unsigned)((n_lanes + BLOCK - 1) / BLOCK);
-   hipLaunchKernelGGL((gc_service<R, BG>), dim3(grid), dim3(BLOCK), 0, st, d_launch);
-   if (mid) {
-      hipError_t e = hipEventRecord(mid, st);
-      if (e != hipSuccess) return e;
+   const unsigned grid = (unsigned)((n_lanes + BLOCK - 1) / BLOCK);   // n_lanes: the slots that may hold a trajectory
+   if constexpr (M != LAUNCH_FEW) {
+      hipLaunchKernelGGL((gc_service<R, BG>), dim3(grid), dim3(BLOCK), 0, st, d_launch);
+      if (mid) {
+         hipError_t e = hipEventRecord(mid, st);
+         if (e != hipSuccess) return e;
+      }
    }
-   hipLaunchKernelGGL((gc_step_kernel<R, BG, XD>), dim3(grid), dim3(BLOCK), 0, st, d_launch);
+   if constexpr (M != LAUNCH_SERVICE)
+      hipLaunchKernelGGL((gc_step_kernel<R, BG, XD, (M == LAUNCH_FEW ? 1 : 0)>), dim3(M == LAUNCH_FEW ? grid * QUAD : grid), dim3(BLOCK), 0, st,
+                         d_launch);
    return hipGetLastError();
 }
 
-template <typename R>
+template <typename R, int M>
 hipError_t dispatch_gc(const spx_plan_desc& hp, uint64_t n_lanes, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
 {
    if (hp.time_flow != 0) return hipErrorInvalidValue;
@@ -691,12 +721,12 @@ hipError_t dispatch_gc(const spx_plan_desc& hp, uint64_t n_lanes, const Launch* 
    const bool xd = (k == SPX_DF_WNLT || k == SPX_DF_WNLT_RAMP || k == SPX_DF_STRAUSS || k == SPX_DF_POTGIETER || k == SPX_DF_SOQLT);
    switch (hp.bg.kind) {
    case SPX_BG_SOLARWIND:
-      return xd ? launch_gc_bg<R, SPX_BG_SOLARWIND, true>(n_lanes, d_launch, st, mid) : launch_gc_bg<R, SPX_BG_SOLARWIND, false>(n_lanes, d_launch, st, mid);
+      return xd ? launch_gc_bg<R, SPX_BG_SOLARWIND, true, M>(n_lanes, d_launch, st, mid) : launch_gc_bg<R, SPX_BG_SOLARWIND, false, M>(n_lanes, d_launch, st, mid);
    case SPX_BG_UNIFORM:
-      return xd ? launch_gc_bg<R, SPX_BG_UNIFORM, true>(n_lanes, d_launch, st, mid) : launch_gc_bg<R, SPX_BG_UNIFORM, false>(n_lanes, d_launch, st, mid);
-   case SPX_BG_GRID: return xd ? hipErrorInvalidValue : launch_gc_bg<R, SPX_BG_GRID, false>(n_lanes, d_launch, st, mid);
-   case SPX_BG_SHOCK: return xd ? hipErrorInvalidValue : launch_gc_bg<R, SPX_BG_SHOCK, false>(n_lanes, d_launch, st, mid);
-   case SPX_BG_SMOOTHSHOCK: return xd ? hipErrorInvalidValue : launch_gc_bg<R, SPX_BG_SMOOTHSHOCK, false>(n_lanes, d_launch, st, mid);
+      return xd ? launch_gc_bg<R, SPX_BG_UNIFORM, true, M>(n_lanes, d_launch, st, mid) : launch_gc_bg<R, SPX_BG_UNIFORM, false, M>(n_lanes, d_launch, st, mid);
+   case SPX_BG_GRID: return xd ? hipErrorInvalidValue : launch_gc_bg<R, SPX_BG_GRID, false, M>(n_lanes, d_launch, st, mid);
+   case SPX_BG_SHOCK: return xd ? hipErrorInvalidValue : launch_gc_bg<R, SPX_BG_SHOCK, false, M>(n_lanes, d_launch, st, mid);
+   case SPX_BG_SMOOTHSHOCK: return xd ? hipErrorInvalidValue : launch_gc_bg<R, SPX_BG_SMOOTHSHOCK, false, M>(n_lanes, d_launch, st, mid);
    default: return hipErrorInvalidValue;
    }
 }

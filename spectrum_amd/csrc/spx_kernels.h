@@ -79,11 +79,27 @@ struct Launch {
 // Host-side dispatch.  One engine launch is the service kernel followed by the step kernel on
 // `stream`; when `mid` is not null it is recorded between the two, so the caller can time each
 // kernel with events.  launch_f64 / launch_f32 pick the instantiation for (transport, background,
-// flow, diffusion) of each precision; they live in separately compiled units.
-hipError_t launch_f64(const spx_plan_desc& host_plan, uint64_t n_lanes, const Launch* dev_launch,
+// flow, diffusion) of each precision; they live in separately compiled units.  The step kernels of has_few exist in
+// two forms with the same results: one for a device full of waves, and one for few resident waves (`few`, in units of
+// their own), where a launch lasts as long as the longest step chain of one wave and most of the chip idles.
+// A wave then issues one instruction every 4 cycles whatever its independence, so the way to a shorter step is
+// fewer instructions per lane: four lanes share a trajectory (quad_get in spx_engine.h).
+enum { LAUNCH_BOTH = 0, LAUNCH_FEW = 1, LAUNCH_SERVICE = 2 };   // dispatch templates: service + step, the few-wave step, service alone
+hipError_t launch_f64(const spx_plan_desc& host_plan, uint64_t n_lanes, const Launch* dev_launch, bool few,
                       hipStream_t stream, hipEvent_t mid);
-hipError_t launch_f32(const spx_plan_desc& host_plan, uint64_t n_lanes, const Launch* dev_launch,
+hipError_t launch_f32(const spx_plan_desc& host_plan, uint64_t n_lanes, const Launch* dev_launch, bool few,
                       hipStream_t stream, hipEvent_t mid);
+hipError_t launch_few_f64(const spx_plan_desc& host_plan, uint64_t n_lanes, const Launch* dev_launch, hipStream_t stream);
+hipError_t launch_few_f32(const spx_plan_desc& host_plan, uint64_t n_lanes, const Launch* dev_launch, hipStream_t stream);
+// Which step kernels have the few-wave form.  Measured on one wave per SIMD, one pass: FP64 modulation 15.6 -> 9.4 ms
+// (64 trajectories), guiding centre 265 -> 189 ms (5000), gridded wind with anisotropic kappa 565 -> 306 ms (10^4);
+// FP32 with kappa ~ T r^2 41 -> 26 ms (2000), gridded anisotropic 289 -> 134 ms (500).
+inline bool has_few(const spx_plan_desc& p, int precision)
+{
+   if (precision == SPX_PREC_FP64) return p.traj_type <= SPX_TRAJ_FIELDLINE;
+   const bool parker = p.traj_type == SPX_TRAJ_PARKER || p.traj_type == SPX_TRAJ_PARKER_SOURCE || p.traj_type == SPX_TRAJ_FIELDLINE;
+   return parker && (p.bg.kind == SPX_BG_SOLARWIND || p.bg.kind == SPX_BG_GRID);
+}
 
 // FP32 cell records of a Cartesian grid (spx_grid_desc::c32) from its device zone records (nz[0] x nz[1] x
 // nz[2], x fastest, SPX_GRID_REC doubles each): for every zone, the 8 zones of the stencil whose lowest
@@ -91,10 +107,10 @@ hipError_t launch_f32(const spx_plan_desc& host_plan, uint64_t n_lanes, const La
 hipError_t grid_expand_cells(const double* zones, const int32_t nz[3], float* c32, hipStream_t st);
 
 inline hipError_t launch_transport(const spx_plan_desc& host_plan, uint64_t n_lanes, const Launch* dev_launch,
-                                   int precision, hipStream_t stream, hipEvent_t mid)
+                                   int precision, bool few, hipStream_t stream, hipEvent_t mid)
 {
-   return precision == SPX_PREC_MIXED ? launch_f32(host_plan, n_lanes, dev_launch, stream, mid)
-                                      : launch_f64(host_plan, n_lanes, dev_launch, stream, mid);
+   return precision == SPX_PREC_MIXED ? launch_f32(host_plan, n_lanes, dev_launch, few, stream, mid)
+                                      : launch_f64(host_plan, n_lanes, dev_launch, few, stream, mid);
 }
 
 }  // namespace spx

@@ -35,11 +35,17 @@ hipError_t grid_expand_cells(const double* zones, const int32_t nz[3], float* c3
    return hipGetLastError();
 }
 
-hipError_t launch_f64(const spx_plan_desc& hp, uint64_t n_lanes, const Launch* d_launch, hipStream_t st,
-                      hipEvent_t mid)
+hipError_t launch_f64(const spx_plan_desc& hp, uint64_t n_lanes, const Launch* d_launch, bool few, hipStream_t st, hipEvent_t mid)
 {
-   if (hp.traj_type == SPX_TRAJ_PARKER || hp.traj_type == SPX_TRAJ_PARKER_SOURCE || hp.traj_type == SPX_TRAJ_FIELDLINE) return dispatch_parker<double>(hp, n_lanes, d_launch, st, mid);
-   if (hp.traj_type >= SPX_TRAJ_GUIDING_DIFF_SCATT && hp.traj_type <= SPX_TRAJ_GUIDING_DIFF) return dispatch_gc<double>(hp, n_lanes, d_launch, st, mid);
+   const bool parker = hp.traj_type == SPX_TRAJ_PARKER || hp.traj_type == SPX_TRAJ_PARKER_SOURCE || hp.traj_type == SPX_TRAJ_FIELDLINE;
+   const bool gc = hp.traj_type >= SPX_TRAJ_GUIDING_DIFF_SCATT && hp.traj_type <= SPX_TRAJ_GUIDING_DIFF;
+   if (few && has_few(hp, SPX_PREC_FP64)) {
+      const hipError_t e = parker ? dispatch_parker<double, LAUNCH_SERVICE>(hp, n_lanes, d_launch, st, mid)
+                                  : dispatch_gc<double, LAUNCH_SERVICE>(hp, n_lanes, d_launch, st, mid);
+      return e != hipSuccess ? e : launch_few_f64(hp, n_lanes, d_launch, st);
+   }
+   if (parker) return dispatch_parker<double, LAUNCH_BOTH>(hp, n_lanes, d_launch, st, mid);
+   if (gc) return dispatch_gc<double, LAUNCH_BOTH>(hp, n_lanes, d_launch, st, mid);
    if (hp.traj_type == SPX_TRAJ_LORENTZ) return dispatch_lorentz<double>(hp, n_lanes, d_launch, st, mid);
    if (hp.traj_type == SPX_TRAJ_FOCUSED) return dispatch_focused<double>(hp, n_lanes, d_launch, st, mid);
    return hipErrorInvalidValue;

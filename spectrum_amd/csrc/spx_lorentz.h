@@ -23,8 +23,8 @@ struct LzFields {
 
 // GetFields with the mask E | B at a position: B, |B| (an ExFieldError below sp_tiny), E from the kept flow
 // U0 (SolarWind) or the uniform field's E, and dmax.
-template <typename R, int BG>
-__device__ __forceinline__ bool lz_fields(const SPX_CP spx_bg_t<R>& bg, double t, double x, double y, double z, v3<R> U0, LzFields<R>& F)
+template <typename R, int BG, typename BD>
+__device__ __forceinline__ bool lz_fields(BD& bg, double t, double x, double y, double z, v3<R> U0, LzFields<R>& F)
 {
    F.dmax = bg_dmax<R, BG>(bg, x, y, z, R(0));
    if constexpr (BG == SPX_BG_GRID) {
@@ -76,7 +76,7 @@ template <typename R, int BG>
 __device__ int lz_set_start(PlanPtr P, QueryPtr Q, LaunchPtr L, const spx_rng_desc& rng, uint64_t slot,
                             uint64_t traj, uint32_t& nu)
 {
-   const SPX_CP spx_bg_t<R>& bg = PlanView<R>::bg(P);
+   auto& bg = PlanView<R>::bg(P);
    const uint64_t first = Q->first;
    const double t = P->it_t;
    bool ex = false;
@@ -150,7 +150,7 @@ struct LzHot {
 template <typename R, int BG, int FWD>
 __device__ __forceinline__ int lz_step(PlanPtr P, LaunchPtr L, uint64_t slot, LzHot<R>& H, ColdLDS& C, int tid, int& bflags)
 {
-   const SPX_CP spx_bg_t<R>& bg = PlanView<R>::bg(P);
+   auto& bg = PlanView<R>::bg(P);
    const v3<R> mom = mk<R>(R(H.px), R(H.py), R(H.pz));
    const R mm = norm(mom);
    const R a = VelP(mm) / mm;
@@ -173,7 +173,7 @@ __device__ __forceinline__ int lz_step(PlanPtr P, LaunchPtr L, uint64_t slot, Lz
       H.x -= (double)(dtv * vel.x); H.y -= (double)(dtv * vel.y); H.z -= (double)(dtv * vel.z);
       H.px -= (double)(dtv * force.x); H.py -= (double)(dtv * force.y); H.pz -= (double)(dtv * force.z);
    }
-   bflags = handle_boundaries<true>(P, L, slot, H, C, tid);
+   bflags = handle_boundaries<true>(P, P, L, slot, H, C, tid);
    if (!(bflags & 1)) {
       if (!lz_fields<R, BG>(bg, H.t, H.x, H.y, H.z, H.U0, H.F)) return 1;
    }

@@ -32,8 +32,8 @@ struct PkFields {
 // src/background_base.cc:425-456, with NumericalDerivatives :228-312 for SolarWind and the analytic
 // derivatives of src/background_smooth_shock.cc:159-187).  The transport consumes only div(U) of the
 // gradients, so only U is evaluated at the derivative points.  Returns false on ExFieldError.
-template <typename R, int BG>
-__device__ __forceinline__ bool parker_fields(const SPX_CP spx_bg_t<R>& bg, double t, double x, double y, double z, R p, R& ds_prev, PkFields<R>& F)
+template <typename R, int BG, int V = 0, typename BD>
+__device__ __forceinline__ bool parker_fields(BD& bg, double t, double x, double y, double z, R p, R& ds_prev, PkFields<R>& F)
 {
    F.dmax = bg_dmax<R, BG>(bg, x, y, z, ds_prev);
    if constexpr (BG == SPX_BG_GRID) {
@@ -80,6 +80,24 @@ __device__ __forceinline__ bool parker_fields(const SPX_CP spx_bg_t<R>& bg, doub
          F.divU = (R(0.5) / r_g) * sw_divu_stencil<R>(bg, dc, r_g, fa);
          return true;
       }
+      if constexpr (V == 1) {   // each lane of the quad takes one axis; the terms are added in the same order
+         const int q = quad_lane();
+         const v3<R> e = q == 0 ? fa[0] : (q == 1 ? fa[1] : fa[2]);
+         R dr = r_g;
+         v3<R> Uf, Ub, Bd;
+         R dsd;
+         const double xf = x + (double)(dr * e.x), yf = y + (double)(dr * e.y), zf = z + (double)(dr * e.z);
+         bg_eval<R, BG>(bg, t, xf, yf, zf, 1, Uf, Bd, dsd);
+         dr *= R(2);
+         bg_eval<R, BG>(bg, t, xf - (double)(dr * e.x), yf - (double)(dr * e.y), zf - (double)(dr * e.z), 1, Ub, Bd, dsd);
+         const v3<R> G = (Uf - Ub) / dr;
+         const R g0 = e.x * G.x, g1 = e.y * G.y, g2 = e.z * G.z;
+         d0 = quad_get<0>(g0) + quad_get<1>(g0) + quad_get<2>(g0);
+         d1 = quad_get<0>(g1) + quad_get<1>(g1) + quad_get<2>(g1);
+         d2 = quad_get<0>(g2) + quad_get<1>(g2) + quad_get<2>(g2);
+         F.divU = d0 + d1 + d2;
+         return true;
+      }
       // the frame vectors rotate through e (moves instead of a select of each component per point)
       v3<R> e = fa[0], e_next = fa[1];
 #pragma unroll 1
@@ -121,8 +139,8 @@ __device__ __forceinline__ bool parker_fields(const SPX_CP spx_bg_t<R>& bg, doub
 // the other analytic backgrounds set positive regions only (src/background_uniform.cc:68,
 // src/background_shock.cc:99-107, src/background_smooth_shock.cc:151).  r is the norm in the rotated frame;
 // the diagonal +-1 bases leave it unchanged.
-template <typename R, int BG>
-__device__ __forceinline__ bool lism_outer(const SPX_CP spx_bg_t<R>& bg, const SPX_CP spx_df_t<R>& df, double x, double y, double z)
+template <typename R, int BG, typename BD, typename DD>
+__device__ __forceinline__ bool lism_outer(BD& bg, DD& df, double x, double y, double z)
 {
    if (BG != SPX_BG_SOLARWIND || df.region_idx < 0) return false;
    if (df.region_idx == 1) return true;
@@ -139,8 +157,8 @@ __device__ __forceinline__ bool lism_outer(const SPX_CP spx_bg_t<R>& bg, const S
 // DiffusionBase::GetComponent for components 0 and 1 at a position.  DF is the diffusion class when it
 // is known at compile time (0 = any, dispatched at run time); km2 is the LISM factor of the region models,
 // or with km3 the two perpendicular factors of the empirical SOQLT model (lam_perp, lam_perp kap_rat_red).
-template <typename R, int BG, int DF>
-__device__ __forceinline__ void parker_kappa(const SPX_CP spx_bg_t<R>& bg, const SPX_CP spx_df_t<R>& df, R km, R km2, R km3, R Bmag,
+template <typename R, int BG, int DF, typename BD, typename DD>
+__device__ __forceinline__ void parker_kappa(BD& bg, DD& df, R km, R km2, R km3, R Bmag,
                                              double x, double y, double z, v3<R> U, R& K0, R& K1)
 {
    if (DF == SPX_DF_RIGBMAG) {   // src/diffusion_other.cc:804-809; pow(x, 0) == 1 exactly
@@ -200,7 +218,7 @@ template <typename R, int BG, int TT>
 __device__ int parker_set_start(PlanPtr P, QueryPtr Q, LaunchPtr L, const spx_rng_desc& rng, uint64_t slot,
                                 uint64_t traj, uint32_t& nu)
 {
-   const SPX_CP spx_bg_t<R>& bg = PlanView<R>::bg(P);
+   auto& bg = PlanView<R>::bg(P);
    const uint64_t first = Q->first;
    const double t = P->it_t;
    bool ex = false;
@@ -256,14 +274,14 @@ __global__ __launch_bounds__(BLOCK) void parker_service(const Launch* __restrict
 }
 
 // ---- step kernel -----------------------------------------------------------------------------
-template <typename R>
+template <typename R, int V>
 struct PkHot {
    double t, x, y, z, p;
    PkFields<R> F;
    R ds_prev;                                   // BackgroundSmoothShock's hidden coordinate (smooth shock only)
    double bd[SPX_MAX_BND], bdo[SPX_MAX_BND];    // boundary _delta and _delta_old
    int bst[SPX_MAX_BND];                        // boundary status bits
-   NormalStream<R> rs;
+   typename StreamOf<R, V>::type rs;
    int32_t steps;
    bool fieldline;                              // TrajectoryFieldline: p is the signed p_par of (0, 0, p_par)
    typedef R real;
@@ -279,10 +297,10 @@ struct PkHot {
 // src/trajectory_base.cc:545-579): the centre follows the magnetic field, slope = v_par bhat with v_par the
 // third component of Particle::Vel(0, 0, p_par) (common/physics.hh:330-336), PhysicalStep
 // dt = 0.5 dmax / |v_par|; the momentum is constant and no random numbers are drawn.
-template <typename R, int BG, int FWD>
-__device__ __forceinline__ int fieldline_step(PlanPtr P, LaunchPtr L, uint64_t slot, PkHot<R>& H, ColdLDS& C, int tid, int& bflags)
+template <typename R, int BG, int FWD, int V, typename PP>
+__device__ __forceinline__ int fieldline_step(PP P, PlanPtr Pc, LaunchPtr L, uint64_t slot, PkHot<R, V>& H, ColdLDS& C, int tid, int& bflags)
 {
-   const SPX_CP spx_bg_t<R>& bg = PlanView<R>::bg(P);
+   auto& bg = PlanView<R>::bg(P);
    const R p = R(H.p), pm = fabs(p);
    const R v = p * (VelP(pm) / pm);
    const R dtp = R(0.5) * H.F.dmax / fabs(v);
@@ -305,9 +323,9 @@ __device__ __forceinline__ int fieldline_step(PlanPtr P, LaunchPtr L, uint64_t s
       H.t -= dt;
       H.x -= (double)(dtv * slope_pos.x); H.y -= (double)(dtv * slope_pos.y); H.z -= (double)(dtv * slope_pos.z);
    }
-   bflags = handle_boundaries<false>(P, L, slot, H, C, tid);
+   bflags = handle_boundaries<false, V>(P, Pc, L, slot, H, C, tid);
    if (!(bflags & 1)) {
-      if (!parker_fields<R, BG>(bg, H.t, H.x, H.y, H.z, R(fabs(H.p)), H.ds_prev, H.F)) return 1;
+      if (!parker_fields<R, BG, V>(bg, H.t, H.x, H.y, H.z, R(fabs(H.p)), H.ds_prev, H.F)) return 1;
    }
    H.steps++;
    if (H.steps > P->max_steps) return 4;
@@ -319,12 +337,12 @@ __device__ __forceinline__ int fieldline_step(PlanPtr P, LaunchPtr L, uint64_t s
 // One Parker step: TrajectoryParker::Advance (src/trajectory_parker.cc:255-306) with the Euler table
 // (common/rk_config.hh:72-80) and TrajectoryBase::Integrate's checks (src/trajectory_base.cc:964-992).
 // Returns an exception code; `bflags` gets handle_boundaries' result.
-template <typename R, int BG, int FWD, int TT, int DF>
-__device__ __forceinline__ int parker_step(PlanPtr P, LaunchPtr L, const spx_rng_desc& rng,
-                                           uint64_t first, uint64_t slot, PkHot<R>& H, ColdLDS& C, int tid, int& bflags)
+template <typename R, int BG, int FWD, int TT, int DF, int V, typename PP>
+__device__ __forceinline__ int parker_step(PP P, PlanPtr Pc, LaunchPtr L, const spx_rng_desc& rng,
+                                           uint64_t first, uint64_t slot, PkHot<R, V>& H, ColdLDS& C, int tid, int& bflags)
 {
-   const SPX_CP spx_bg_t<R>& bg = PlanView<R>::bg(P);
-   const SPX_CP spx_df_t<R>& df = PlanView<R>::df(P);
+   auto& bg = PlanView<R>::bg(P);
+   auto& df = PlanView<R>::df(P);
    const R p = R(H.p);
    // DriftCoeff + DiffusionCoeff (src/trajectory_parker.cc:189-206, 83-153)
    R K0 = R(0), K1 = R(0);
@@ -343,8 +361,7 @@ __device__ __forceinline__ int parker_step(PlanPtr P, LaunchPtr L, const spx_rng
    const bool pos_dep = (DF == SPX_DF_FULL) ? false : (df.pos_dep != 0);
    if (BG == SPX_BG_GRID && (pos_dep || K0 != K1)) {
       // the same stencil on the gridded background: interpolated B and |B| at the derivative points
-#pragma unroll 1
-      for (int j = 0; j < 3; j++) {
+      auto axis = [&](int j, v3<R>& t) -> bool {
          const double ex = (j == 0) ? 1.0 : 0.0, ey = (j == 1) ? 1.0 : 0.0, ez = (j == 2) ? 1.0 : 0.0;
          double xf = H.x + (double)delta * ex, yf = H.y + (double)delta * ey, zf = H.z + (double)delta * ez;
          // with fd_fields == 0 the fields at these points cannot change the result (the host has shown it):
@@ -353,48 +370,80 @@ __device__ __forceinline__ int parker_step(PlanPtr P, LaunchPtr L, const spx_rng
          GridFields<R> Gf, Gb;
          Gf.U = Gb.U = Gf.B = Gb.B = mk<R>(R(0), R(0), R(0));
          Gf.Bmag = Gb.Bmag = H.F.Bmag;
-         if (loads ? !grid_eval<R, false>(bg.grid, xf, yf, zf, Gf) : !grid_inside<R>(bg.grid, xf, yf, zf)) return 1;
-         if (loads && Gf.Bmag < R(sp_tiny)) return 1;
+         if (loads ? !grid_eval<R, false>(bg.grid, xf, yf, zf, Gf) : !grid_inside<R>(bg.grid, xf, yf, zf)) return false;
+         if (loads && Gf.Bmag < R(sp_tiny)) return false;
          const v3<R> bf = !loads ? Gf.B : (is_f32<R>() ? (R(1) / Gf.Bmag) * Gf.B : Gf.B / Gf.Bmag);
          R K0f = K0, K1f = K1;
          if (pos_dep) parker_kappa<R, BG, DF>(bg, df, km, km2, km3, Gf.Bmag, xf, yf, zf, Gf.U, K0f, K1f);
          xf -= 2.0 * (double)delta * ex;
          yf -= 2.0 * (double)delta * ey;
          zf -= 2.0 * (double)delta * ez;
-         if (loads ? !grid_eval<R, false>(bg.grid, xf, yf, zf, Gb) : !grid_inside<R>(bg.grid, xf, yf, zf)) return 1;
-         if (loads && Gb.Bmag < R(sp_tiny)) return 1;
+         if (loads ? !grid_eval<R, false>(bg.grid, xf, yf, zf, Gb) : !grid_inside<R>(bg.grid, xf, yf, zf)) return false;
+         if (loads && Gb.Bmag < R(sp_tiny)) return false;
          const v3<R> bb = !loads ? Gb.B : (is_f32<R>() ? (R(1) / Gb.Bmag) * Gb.B : Gb.B / Gb.Bmag);
          R K0b = K0, K1b = K1;
          if (pos_dep) parker_kappa<R, BG, DF>(bg, df, km, km2, km3, Gb.Bmag, xf, yf, zf, Gb.U, K0b, K1b);
          const R bfj = j == 0 ? bf.x : (j == 1 ? bf.y : bf.z);
          const R bbj = j == 0 ? bb.x : (j == 1 ? bb.y : bb.z);
          const R cf = (K1f - K0f) * bfj, cb = (K1b - K0b) * bbj;
+         t = mk<R>((K0f * (j == 0 ? R(1) : R(0)) + cf * bf.x) - (K0b * (j == 0 ? R(1) : R(0)) + cb * bb.x),
+                   (K0f * (j == 1 ? R(1) : R(0)) + cf * bf.y) - (K0b * (j == 1 ? R(1) : R(0)) + cb * bb.y),
+                   (K0f * (j == 2 ? R(1) : R(0)) + cf * bf.z) - (K0b * (j == 2 ? R(1) : R(0)) + cb * bb.z));
+         return true;
+      };
+      auto add = [&](v3<R> t) {
          if constexpr (is_f32<R>()) {   // one reciprocal of delta for the whole stencil
-            divK.x += hdi * ((K0f * (j == 0 ? R(1) : R(0)) + cf * bf.x) - (K0b * (j == 0 ? R(1) : R(0)) + cb * bb.x));
-            divK.y += hdi * ((K0f * (j == 1 ? R(1) : R(0)) + cf * bf.y) - (K0b * (j == 1 ? R(1) : R(0)) + cb * bb.y));
-            divK.z += hdi * ((K0f * (j == 2 ? R(1) : R(0)) + cf * bf.z) - (K0b * (j == 2 ? R(1) : R(0)) + cb * bb.z));
+            divK.x += hdi * t.x;
+            divK.y += hdi * t.y;
+            divK.z += hdi * t.z;
          }
          else {
-            divK.x += div_rn(R(0.5) * ((K0f * (j == 0 ? R(1) : R(0)) + cf * bf.x) - (K0b * (j == 0 ? R(1) : R(0)) + cb * bb.x)), delta, ydel);
-            divK.y += div_rn(R(0.5) * ((K0f * (j == 1 ? R(1) : R(0)) + cf * bf.y) - (K0b * (j == 1 ? R(1) : R(0)) + cb * bb.y)), delta, ydel);
-            divK.z += div_rn(R(0.5) * ((K0f * (j == 2 ? R(1) : R(0)) + cf * bf.z) - (K0b * (j == 2 ? R(1) : R(0)) + cb * bb.z)), delta, ydel);
+            divK.x += div_rn(R(0.5) * t.x, delta, ydel);
+            divK.y += div_rn(R(0.5) * t.y, delta, ydel);
+            divK.z += div_rn(R(0.5) * t.z, delta, ydel);
+         }
+      };
+      if constexpr (V == 1) {   // an axis per lane of the quad, added in the same order
+         v3<R> t = mk<R>(R(0), R(0), R(0));
+         if (quad_any(!axis(min(quad_lane(), 2), t))) return 1;
+         add(mk<R>(quad_get<0>(t.x), quad_get<0>(t.y), quad_get<0>(t.z)));
+         own_rounding(divK);
+         add(mk<R>(quad_get<1>(t.x), quad_get<1>(t.y), quad_get<1>(t.z)));
+         own_rounding(divK);
+         add(mk<R>(quad_get<2>(t.x), quad_get<2>(t.y), quad_get<2>(t.z)));
+         own_rounding(divK);
+      }
+      else {
+#pragma unroll 1
+         for (int j = 0; j < 3; j++) {
+            v3<R> t;
+            if (!axis(j, t)) return 1;
+            add(t);
          }
       }
    }
    else if (BG == SPX_BG_GRID) {
       // divK vanishes identically, but the reference still evaluates the six derivative points, and one
       // outside the grid discards the attempt
-#pragma unroll 1
-      for (int j = 0; j < 3; j++) {
+      auto axis = [&](int j) -> bool {
          const double ex = (j == 0) ? 1.0 : 0.0, ey = (j == 1) ? 1.0 : 0.0, ez = (j == 2) ? 1.0 : 0.0;
          double xf = H.x + (double)delta * ex, yf = H.y + (double)delta * ey, zf = H.z + (double)delta * ez;
          const bool loads = bg.grid.fd_fields != 0;
          GridFields<R> G;
-         if (loads ? (!grid_eval<R, false>(bg.grid, xf, yf, zf, G) || G.Bmag < R(sp_tiny)) : !grid_inside<R>(bg.grid, xf, yf, zf)) return 1;
+         if (loads ? (!grid_eval<R, false>(bg.grid, xf, yf, zf, G) || G.Bmag < R(sp_tiny)) : !grid_inside<R>(bg.grid, xf, yf, zf)) return false;
          xf -= 2.0 * (double)delta * ex;
          yf -= 2.0 * (double)delta * ey;
          zf -= 2.0 * (double)delta * ez;
-         if (loads ? (!grid_eval<R, false>(bg.grid, xf, yf, zf, G) || G.Bmag < R(sp_tiny)) : !grid_inside<R>(bg.grid, xf, yf, zf)) return 1;
+         if (loads ? (!grid_eval<R, false>(bg.grid, xf, yf, zf, G) || G.Bmag < R(sp_tiny)) : !grid_inside<R>(bg.grid, xf, yf, zf)) return false;
+         return true;
+      };
+      if constexpr (V == 1) {
+         if (quad_any(!axis(min(quad_lane(), 2)))) return 1;
+      }
+      else {
+#pragma unroll 1
+         for (int j = 0; j < 3; j++)
+            if (!axis(j)) return 1;
       }
    }
    else if (is_f32<R>() && BG == SPX_BG_SOLARWIND && !pos_dep && K0 != K1 && bg.ep_diag != 0 &&
@@ -407,8 +456,8 @@ __device__ __forceinline__ int parker_step(PlanPtr P, LaunchPtr L, const spx_rng
       // FP32 steps with a position-independent kappa evaluate the stencil relative to the origin
       v3<R> dc = mk<R>(R(0), R(0), R(0));
       if constexpr (is_f32<R>()) dc = rel(bg, H.x, H.y, H.z);
-#pragma unroll 1
-      for (int j = 0; j < 3; j++) {
+      R ds_last = H.ds_prev;
+      auto axis = [&](int j, v3<R>& t) -> bool {
          const double ex = (j == 0) ? 1.0 : 0.0, ey = (j == 1) ? 1.0 : 0.0, ez = (j == 2) ? 1.0 : 0.0;
          const v3<R> ej = mk<R>(R(ex), R(ey), R(ez));
          double xf = H.x + (double)delta * ex, yf = H.y + (double)delta * ey, zf = H.z + (double)delta * ez;
@@ -420,7 +469,7 @@ __device__ __forceinline__ int parker_step(PlanPtr P, LaunchPtr L, const spx_rng
          v3<R> bf;
          if constexpr (is_f32<R>()) { const R b2 = norm2(B2), ib = frsq(b2); Bmf = b2 * ib; bf = ib * B2; }
          else { Bmf = norm(B2); bf = B2 / Bmf; }
-         if (Bmf < R(sp_tiny)) return 1;
+         if (Bmf < R(sp_tiny)) return false;
          R K0f = K0, K1f = K1;
          if (pos_dep) parker_kappa<R, BG, DF>(bg, df, km, km2, km3, Bmf, xf, yf, zf, U2, K0f, K1f);
          xf -= 2.0 * (double)delta * ex;
@@ -428,27 +477,53 @@ __device__ __forceinline__ int parker_step(PlanPtr P, LaunchPtr L, const spx_rng
          zf -= 2.0 * (double)delta * ez;
          if (is_f32<R>() && !pos_dep) bg_eval_rel<R, BG>(bg, H.t, dc + delta * ej - (R(2) * delta) * ej, want, U2, B2, dsd);
          else bg_eval<R, BG>(bg, H.t, xf, yf, zf, want, U2, B2, dsd);
-         if (BG == SPX_BG_SMOOTHSHOCK) H.ds_prev = dsd;
+         if (BG == SPX_BG_SMOOTHSHOCK) ds_last = dsd;
          R Bmb;
          v3<R> bb;
          if constexpr (is_f32<R>()) { const R b2 = norm2(B2), ib = frsq(b2); Bmb = b2 * ib; bb = ib * B2; }
          else { Bmb = norm(B2); bb = B2 / Bmb; }
-         if (Bmb < R(sp_tiny)) return 1;
+         if (Bmb < R(sp_tiny)) return false;
          R K0b = K0, K1b = K1;
          if (pos_dep) parker_kappa<R, BG, DF>(bg, df, km, km2, km3, Bmb, xf, yf, zf, U2, K0b, K1b);
          const R bfj = j == 0 ? bf.x : (j == 1 ? bf.y : bf.z);
          const R bbj = j == 0 ? bb.x : (j == 1 ? bb.y : bb.z);
          const R cf = (K1f - K0f) * bfj, cb = (K1b - K0b) * bbj;
+         t = mk<R>((K0f * (j == 0 ? R(1) : R(0)) + cf * bf.x) - (K0b * (j == 0 ? R(1) : R(0)) + cb * bb.x),
+                   (K0f * (j == 1 ? R(1) : R(0)) + cf * bf.y) - (K0b * (j == 1 ? R(1) : R(0)) + cb * bb.y),
+                   (K0f * (j == 2 ? R(1) : R(0)) + cf * bf.z) - (K0b * (j == 2 ? R(1) : R(0)) + cb * bb.z));
+         return true;
+      };
+      auto add = [&](v3<R> t) {
          if constexpr (is_f32<R>()) {   // one reciprocal of delta for the whole stencil
-            divK.x += hdi * ((K0f * (j == 0 ? R(1) : R(0)) + cf * bf.x) - (K0b * (j == 0 ? R(1) : R(0)) + cb * bb.x));
-            divK.y += hdi * ((K0f * (j == 1 ? R(1) : R(0)) + cf * bf.y) - (K0b * (j == 1 ? R(1) : R(0)) + cb * bb.y));
-            divK.z += hdi * ((K0f * (j == 2 ? R(1) : R(0)) + cf * bf.z) - (K0b * (j == 2 ? R(1) : R(0)) + cb * bb.z));
+            divK.x += hdi * t.x;
+            divK.y += hdi * t.y;
+            divK.z += hdi * t.z;
          }
          else {
-            divK.x += div_rn(R(0.5) * ((K0f * (j == 0 ? R(1) : R(0)) + cf * bf.x) - (K0b * (j == 0 ? R(1) : R(0)) + cb * bb.x)), delta, ydel);
-            divK.y += div_rn(R(0.5) * ((K0f * (j == 1 ? R(1) : R(0)) + cf * bf.y) - (K0b * (j == 1 ? R(1) : R(0)) + cb * bb.y)), delta, ydel);
-            divK.z += div_rn(R(0.5) * ((K0f * (j == 2 ? R(1) : R(0)) + cf * bf.z) - (K0b * (j == 2 ? R(1) : R(0)) + cb * bb.z)), delta, ydel);
+            divK.x += div_rn(R(0.5) * t.x, delta, ydel);
+            divK.y += div_rn(R(0.5) * t.y, delta, ydel);
+            divK.z += div_rn(R(0.5) * t.z, delta, ydel);
          }
+      };
+      if constexpr (V == 1) {   // an axis per lane of the quad, added in the same order
+         v3<R> t = mk<R>(R(0), R(0), R(0));
+         if (quad_any(!axis(min(quad_lane(), 2), t))) return 1;
+         add(mk<R>(quad_get<0>(t.x), quad_get<0>(t.y), quad_get<0>(t.z)));
+         own_rounding(divK);
+         add(mk<R>(quad_get<1>(t.x), quad_get<1>(t.y), quad_get<1>(t.z)));
+         own_rounding(divK);
+         add(mk<R>(quad_get<2>(t.x), quad_get<2>(t.y), quad_get<2>(t.z)));
+         own_rounding(divK);
+         if (BG == SPX_BG_SMOOTHSHOCK) H.ds_prev = quad_get<2>(ds_last);
+      }
+      else {
+#pragma unroll 1
+         for (int j = 0; j < 3; j++) {
+            v3<R> t;
+            if (!axis(j, t)) return 1;
+            add(t);
+         }
+         if (BG == SPX_BG_SMOOTHSHOCK) H.ds_prev = ds_last;
       }
    }
    else if (BG == SPX_BG_SMOOTHSHOCK) {
@@ -515,9 +590,9 @@ __device__ __forceinline__ int parker_step(PlanPtr P, LaunchPtr L, const spx_rng
       C.dt_prev[tid] = dt;
    }
    // HandleBoundaries and the end-of-step fields
-   bflags = handle_boundaries<false>(P, L, slot, H, C, tid);
+   bflags = handle_boundaries<false, V>(P, Pc, L, slot, H, C, tid);
    if (!(bflags & 1)) {
-      if (!parker_fields<R, BG>(bg, H.t, H.x, H.y, H.z, R(H.p), H.ds_prev, H.F)) return 1;
+      if (!parker_fields<R, BG, V>(bg, H.t, H.x, H.y, H.z, R(H.p), H.ds_prev, H.F)) return 1;
    }
    H.steps++;
    // Integrate's safety checks
@@ -527,13 +602,15 @@ __device__ __forceinline__ int parker_step(PlanPtr P, LaunchPtr L, const spx_rng
    return 0;
 }
 
-template <typename R, int BG, int FWD, int TT, int DF>
+template <typename R, int BG, int FWD, int TT, int DF, int V>
 __device__ __forceinline__ void parker_step_body(const Launch* __restrict__ Lg)
 {
    const LaunchPtr Lp = (LaunchPtr)Lg;
    __shared__ ColdLDS C;
    const int tid = threadIdx.x;
-   const uint64_t slot = (uint64_t)blockIdx.x * BLOCK + tid;
+   __shared__ RingLDS<R, V> ring;
+   const uint64_t slot = slot_of<V>();
+   const bool writer = slot_writer<V>();
    // the slots of a wave work for one query (the pool size is a multiple of the block size)
    const int q = __builtin_amdgcn_readfirstlane(Lp->slot_q[slot]);
    const bool run = q >= 0 && Lp->active[slot] == SLOT_RUN;
@@ -542,7 +619,7 @@ __device__ __forceinline__ void parker_step_body(const Launch* __restrict__ Lg)
    const PlanPtr P = plan_of(Q);
    const spx_rng_desc rng = load_rng(Q);
    const uint64_t first = Q->first;
-   PkHot<R> H;
+   PkHot<R, V> H;
    if (run) {
       const uint64_t n = Lp->n_lanes;
       H.fieldline = (TT == 2);
@@ -554,6 +631,7 @@ __device__ __forceinline__ void parker_step_body(const Launch* __restrict__ Lg)
       H.steps = (int32_t)Lp->steps[slot];
       H.ds_prev = R(Lp->ds_prev[slot]);
       H.rs.traj = Lp->traj[slot]; H.rs.nn = Lp->nn[slot]; H.rs.exhausted = false;
+      ring.bind(H.rs);
       prime_normals<R>(rng, H.rs);
       C.amp[tid] = Lp->amp[slot]; C.wgt[tid] = Lp->wgt[slot]; C.dt_adapt[tid] = Lp->dt_adapt[slot];
       C.dt_prev[tid] = Lp->dt_prev[slot]; C.src_old[tid] = Lp->src_old[slot];
@@ -572,18 +650,30 @@ __device__ __forceinline__ void parker_step_body(const Launch* __restrict__ Lg)
    int st = run ? SLOT_RUN : SLOT_IDLE;
    int exc = 0;
    unsigned long long steps_here = 0;
-   for (int it = 0; it < Lp->steps_per_launch; it++) {
+   HotPlan<R> hot;
+   if constexpr (V == 1 && !is_f32<R>()) load_hot(hot, P);
+   const int n_steps = Lp->steps_per_launch;
+   for (int it = 0; it < n_steps; it++) {
       if (__ballot(st == SLOT_RUN) == 0) break;
       if (st != SLOT_RUN) continue;
-      // Re-read the plan and launch block each step instead of pinning their fields in registers: they are
-      // uniform scalar loads, cheap to repeat, while keeping them live would exhaust the register file.
+      int bflags = 0;
+      int e;
+      // V = 0 re-reads the plan and launch block each step instead of pinning their fields in registers: uniform
+      // scalar loads whose latency the other resident waves hide, while keeping them live would exhaust the
+      // register file.  V = 1 runs where few waves are resident and keeps them (HotPlan).
       PlanPtr Pi = P;
       asm volatile("" : "+s"(Pi));
       LaunchPtr Li = Lp;
       asm volatile("" : "+s"(Li));
-      int bflags = 0;
-      const int e = (TT == 2) ? fieldline_step<R, BG, FWD>(Pi, Li, slot, H, C, tid, bflags)
-                              : parker_step<R, BG, FWD, TT, DF>(Pi, Li, rng, first, slot, H, C, tid, bflags);
+      if constexpr (V == 1 && !is_f32<R>()) {
+         const HotPlan<R>* h = &hot;
+         e = (TT == 2) ? fieldline_step<R, BG, FWD, V>(h, Pi, Li, slot, H, C, tid, bflags)
+                       : parker_step<R, BG, FWD, TT, DF, V>(h, Pi, Li, rng, first, slot, H, C, tid, bflags);
+      }
+      else {
+         e = (TT == 2) ? fieldline_step<R, BG, FWD, V>(Pi, Pi, Li, slot, H, C, tid, bflags)
+                       : parker_step<R, BG, FWD, TT, DF, V>(Pi, Pi, Li, rng, first, slot, H, C, tid, bflags);
+      }
       steps_here++;
       if (e != 0) { exc = e; st = SLOT_DISCARD; }
       else if (bflags & 1) st = SLOT_DONE;
@@ -591,10 +681,10 @@ __device__ __forceinline__ void parker_step_body(const Launch* __restrict__ Lg)
    }
    LaunchPtr Ls = Lp;
    asm volatile("" : "+s"(Ls));
-   unsigned long long s = steps_here;
+   unsigned long long s = writer ? steps_here : 0;
    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
    if (lane_id() == 0 && s) atomicAdd(&Q->ctl->steps_executed, s);
-   if (!run) return;
+   if (!run || !writer) return;
    const uint64_t n = Ls->n_lanes;
    Ls->active[slot] = st;
    Ls->ex_code[slot] = exc;
@@ -631,87 +721,88 @@ constexpr int pk_waves()
    return (!is_f32<R>() && BG == SPX_BG_SMOOTHSHOCK && TT == 1 && DF == SPX_DF_FULL) ? 3 : 1;
 #endif
 }
-template <typename R, int BG, int FWD, int TT, int DF>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(pk_waves<R, BG, TT, DF>())))
+template <typename R, int BG, int FWD, int TT, int DF, int V>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(V == 1 ? 1 : pk_waves<R, BG, TT, DF>())))
 void parker_step_kernel(const Launch* __restrict__ Lg)
 {
-   parker_step_body<R, BG, FWD, TT, DF>(Lg);
+   parker_step_body<R, BG, FWD, TT, DF, V>(Lg);
 }
 
-// The gridded background's step kernel waits on gathers: it asks the compiler for room for
-// SPX_GRID_WAVES resident waves per SIMD (0: the compiler's own register budget).
+// The gridded background's step kernel waits on gathers: its V = 0 form asks the compiler for room for
+// SPX_GRID_WAVES resident waves per SIMD (1: the compiler's own register budget).
 #ifndef SPX_GRID_WAVES
-#define SPX_GRID_WAVES 0
+#define SPX_GRID_WAVES 1
 #endif
-#if SPX_GRID_WAVES > 0
-#define SPX_GRID_ATTR __attribute__((amdgpu_waves_per_eu(SPX_GRID_WAVES)))
-#else
-#define SPX_GRID_ATTR
-#endif
-template <typename R, int FWD, int TT>
-__global__ __launch_bounds__(BLOCK) SPX_GRID_ATTR void parker_grid_step_kernel(const Launch* __restrict__ Lg)
+template <typename R, int FWD, int TT, int V>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(V == 1 ? 1 : SPX_GRID_WAVES))) void parker_grid_step_kernel(const Launch* __restrict__ Lg)
 {
-   parker_step_body<R, SPX_BG_GRID, FWD, TT, 0>(Lg);
+   parker_step_body<R, SPX_BG_GRID, FWD, TT, 0, V>(Lg);
 }
 
 // ---------------------------------------------------------------------------------------------
-// Dispatch: one engine launch = service kernel + step kernel on the same stream
+// Dispatch: one engine launch = service kernel + step kernel on the same stream (M: spx_kernels.h)
 // ---------------------------------------------------------------------------------------------
-template <typename R, int BG, int FWD, int TT, int DF>
+template <typename R, int BG, int FWD, int TT, int DF, int M>
 static hipError_t launch_parker(uint64_t n_lanes, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
 {
-   const unsigned grid = (unsigned)((n_lanes + BLOCK - 1) / BLOCK);
-   hipLaunchKernelGGL((parker_service<R, BG, TT>), dim3(grid), dim3(BLOCK), 0, st, d_launch);
-   if (mid) {
-      hipError_t e = hipEventRecord(mid, st);
-      if (e != hipSuccess) return e;
+   const unsigned grid = (unsigned)((n_lanes + BLOCK - 1) / BLOCK);   // n_lanes: the slots that may hold a trajectory
+   if constexpr (M != LAUNCH_FEW) {
+      hipLaunchKernelGGL((parker_service<R, BG, TT>), dim3(grid), dim3(BLOCK), 0, st, d_launch);
+      if (mid) {
+         hipError_t e = hipEventRecord(mid, st);
+         if (e != hipSuccess) return e;
+      }
    }
-   if constexpr (BG == SPX_BG_GRID) hipLaunchKernelGGL((parker_grid_step_kernel<R, FWD, TT>), dim3(grid), dim3(BLOCK), 0, st, d_launch);
-   else hipLaunchKernelGGL((parker_step_kernel<R, BG, FWD, TT, DF>), dim3(grid), dim3(BLOCK), 0, st, d_launch);
+   if constexpr (M != LAUNCH_SERVICE) {
+      constexpr int V = (M == LAUNCH_FEW) ? 1 : 0;
+      const unsigned sg = V == 1 ? grid * QUAD : grid;
+      if constexpr (BG == SPX_BG_GRID) hipLaunchKernelGGL((parker_grid_step_kernel<R, FWD, TT, V>), dim3(sg), dim3(BLOCK), 0, st, d_launch);
+      else hipLaunchKernelGGL((parker_step_kernel<R, BG, FWD, TT, DF, V>), dim3(sg), dim3(BLOCK), 0, st, d_launch);
+   }
    return hipGetLastError();
 }
 
-template <typename R, int BG, int FWD, int TT>
+template <typename R, int BG, int FWD, int TT, int M>
 static hipError_t dispatch_df(const spx_plan_desc& hp, uint64_t n_lanes, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
 {
    switch (hp.df.kind) {
-   case SPX_DF_RIGBMAG: return launch_parker<R, BG, FWD, TT, SPX_DF_RIGBMAG>(n_lanes, d_launch, st, mid);
-   case SPX_DF_FULL: return launch_parker<R, BG, FWD, TT, SPX_DF_FULL>(n_lanes, d_launch, st, mid);
-   default: return launch_parker<R, BG, FWD, TT, 0>(n_lanes, d_launch, st, mid);
+   case SPX_DF_RIGBMAG: return launch_parker<R, BG, FWD, TT, SPX_DF_RIGBMAG, M>(n_lanes, d_launch, st, mid);
+   case SPX_DF_FULL: return launch_parker<R, BG, FWD, TT, SPX_DF_FULL, M>(n_lanes, d_launch, st, mid);
+   default: return launch_parker<R, BG, FWD, TT, 0, M>(n_lanes, d_launch, st, mid);
    }
 }
 
-template <typename R, int BG>
+template <typename R, int BG, int M>
 static hipError_t dispatch_flow(const spx_plan_desc& hp, uint64_t n_lanes, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
 {
    const bool fwd = hp.time_flow == 0;
-   if (hp.traj_type == 1) return fwd ? dispatch_df<R, BG, 1, 1>(hp, n_lanes, d_launch, st, mid) : dispatch_df<R, BG, 0, 1>(hp, n_lanes, d_launch, st, mid);
+   if (hp.traj_type == 1) return fwd ? dispatch_df<R, BG, 1, 1, M>(hp, n_lanes, d_launch, st, mid) : dispatch_df<R, BG, 0, 1, M>(hp, n_lanes, d_launch, st, mid);
    if (hp.traj_type == SPX_TRAJ_FIELDLINE)
-      return fwd ? launch_parker<R, BG, 1, 2, 0>(n_lanes, d_launch, st, mid) : launch_parker<R, BG, 0, 2, 0>(n_lanes, d_launch, st, mid);
-   return fwd ? dispatch_df<R, BG, 1, 0>(hp, n_lanes, d_launch, st, mid) : dispatch_df<R, BG, 0, 0>(hp, n_lanes, d_launch, st, mid);
+      return fwd ? launch_parker<R, BG, 1, 2, 0, M>(n_lanes, d_launch, st, mid) : launch_parker<R, BG, 0, 2, 0, M>(n_lanes, d_launch, st, mid);
+   return fwd ? dispatch_df<R, BG, 1, 0, M>(hp, n_lanes, d_launch, st, mid) : dispatch_df<R, BG, 0, 0, M>(hp, n_lanes, d_launch, st, mid);
 }
 
 // The gridded background runs the generic diffusion dispatch only (every class through kappa01).
-template <typename R>
+template <typename R, int M>
 static hipError_t dispatch_grid(const spx_plan_desc& hp, uint64_t n_lanes, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
 {
    const bool fwd = hp.time_flow == 0;
    constexpr int G = SPX_BG_GRID;
-   if (hp.traj_type == 1) return fwd ? launch_parker<R, G, 1, 1, 0>(n_lanes, d_launch, st, mid) : launch_parker<R, G, 0, 1, 0>(n_lanes, d_launch, st, mid);
+   if (hp.traj_type == 1) return fwd ? launch_parker<R, G, 1, 1, 0, M>(n_lanes, d_launch, st, mid) : launch_parker<R, G, 0, 1, 0, M>(n_lanes, d_launch, st, mid);
    if (hp.traj_type == SPX_TRAJ_FIELDLINE)
-      return fwd ? launch_parker<R, G, 1, 2, 0>(n_lanes, d_launch, st, mid) : launch_parker<R, G, 0, 2, 0>(n_lanes, d_launch, st, mid);
-   return fwd ? launch_parker<R, G, 1, 0, 0>(n_lanes, d_launch, st, mid) : launch_parker<R, G, 0, 0, 0>(n_lanes, d_launch, st, mid);
+      return fwd ? launch_parker<R, G, 1, 2, 0, M>(n_lanes, d_launch, st, mid) : launch_parker<R, G, 0, 2, 0, M>(n_lanes, d_launch, st, mid);
+   return fwd ? launch_parker<R, G, 1, 0, 0, M>(n_lanes, d_launch, st, mid) : launch_parker<R, G, 0, 0, 0, M>(n_lanes, d_launch, st, mid);
 }
 
-template <typename R>
+template <typename R, int M>
 hipError_t dispatch_parker(const spx_plan_desc& hp, uint64_t n_lanes, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
 {
    switch (hp.bg.kind) {
-   case SPX_BG_GRID: return dispatch_grid<R>(hp, n_lanes, d_launch, st, mid);
-   case SPX_BG_SOLARWIND: return dispatch_flow<R, SPX_BG_SOLARWIND>(hp, n_lanes, d_launch, st, mid);
-   case SPX_BG_SMOOTHSHOCK: return dispatch_flow<R, SPX_BG_SMOOTHSHOCK>(hp, n_lanes, d_launch, st, mid);
-   case SPX_BG_SHOCK: return dispatch_flow<R, SPX_BG_SHOCK>(hp, n_lanes, d_launch, st, mid);
-   case SPX_BG_UNIFORM: return dispatch_flow<R, SPX_BG_UNIFORM>(hp, n_lanes, d_launch, st, mid);
+   case SPX_BG_GRID: return dispatch_grid<R, M>(hp, n_lanes, d_launch, st, mid);
+   case SPX_BG_SOLARWIND: return dispatch_flow<R, SPX_BG_SOLARWIND, M>(hp, n_lanes, d_launch, st, mid);
+   case SPX_BG_SMOOTHSHOCK: return dispatch_flow<R, SPX_BG_SMOOTHSHOCK, M>(hp, n_lanes, d_launch, st, mid);
+   case SPX_BG_SHOCK: return dispatch_flow<R, SPX_BG_SHOCK, M>(hp, n_lanes, d_launch, st, mid);
+   case SPX_BG_UNIFORM: return dispatch_flow<R, SPX_BG_UNIFORM, M>(hp, n_lanes, d_launch, st, mid);
    default: return hipErrorInvalidValue;
    }
 }

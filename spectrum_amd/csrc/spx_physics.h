@@ -126,27 +126,105 @@ struct Fields {
 #define SPX_CP __attribute__((address_space(4)))
 typedef const SPX_CP spx_plan_desc* PlanPtr;
 
+// The plan as the FP64 step kernels for few waves keep it: the members a step reads, under the plan's names, copied
+// once per launch into a local object that the compiler splits into scalar registers.  A step that reads the
+// plan through PlanPtr instead waits for a chain of scalar loads (74 in the FP64 modulation step), which other
+// resident waves hide; with one wave per SIMD nothing does (2.4 of 20.3 thousand cycles of that step).  The FP32
+// kernels always read the plan: from a copy the optimizer takes reciprocals of its members out of the loop and lays
+// out other basic blocks, and with contraction across statements the step then rounds differently.
+template <typename R>
+struct HotPlan {
+   int32_t traj_type, n_bnd, n_bt;
+   int64_t max_steps;
+   double dt_scale, src_p_inj, src_rate;
+   spx_bg_t<R> vbg;
+   spx_df_t<R> vdf;
+   spx_bnd_desc bnd[SPX_MAX_BND];
+};
+
 // The descriptors of the step type R.
 template <typename R> struct PlanView;
 template <> struct PlanView<double> {
    static __device__ const SPX_CP spx_bg_t<double>& bg(PlanPtr P) { return P->bg; }
    static __device__ const SPX_CP spx_df_t<double>& df(PlanPtr P) { return P->df; }
+   static __device__ const spx_bg_t<double>& bg(const HotPlan<double>* P) { return P->vbg; }
+   static __device__ const spx_df_t<double>& df(const HotPlan<double>* P) { return P->vdf; }
 };
 template <> struct PlanView<float> {
    static __device__ const SPX_CP spx_bg_t<float>& bg(PlanPtr P) { return P->bgf; }
    static __device__ const SPX_CP spx_df_t<float>& df(PlanPtr P) { return P->dff; }
+   static __device__ const spx_bg_t<float>& bg(const HotPlan<float>* P) { return P->vbg; }
+   static __device__ const spx_df_t<float>& df(const HotPlan<float>* P) { return P->vdf; }
 };
 
+__device__ __forceinline__ const spx_bg_t<double>& hot_bg(const spx_plan_desc* g, double*) { return g->bg; }
+__device__ __forceinline__ const spx_bg_t<float>& hot_bg(const spx_plan_desc* g, float*) { return g->bgf; }
+__device__ __forceinline__ const spx_df_t<double>& hot_df(const spx_plan_desc* g, double*) { return g->df; }
+__device__ __forceinline__ const spx_df_t<float>& hot_df(const spx_plan_desc* g, float*) { return g->dff; }
+// Each member goes through an empty asm: its value is then opaque, so the register allocator cannot repeat the
+// load inside the step loop in place of keeping it.  Members that nothing reads disappear.  Numbers go to vector
+// registers (free where few waves are resident), what branches read to scalar ones.
+__device__ __forceinline__ void opaque(double& d) { asm("" : "+v"(d)); }
+__device__ __forceinline__ void opaque(float& d) { asm("" : "+v"(d)); }
+__device__ __forceinline__ void opaque(int32_t& d) { asm("" : "+s"(d)); }
+__device__ __forceinline__ void opaque(int64_t& d) { asm("" : "+s"(d)); }
+template <typename T> __device__ __forceinline__ void opaque(const T*& d) { asm("" : "+s"(d)); }
+struct HotLoad {
+   template <typename T> __device__ __forceinline__ void operator()(T& d, const T& s) const { d = s; opaque(d); }
+   template <typename T, int N> __device__ __forceinline__ void operator()(T (&d)[N], const T (&s)[N]) const
+   {
+#pragma unroll
+      for (int i = 0; i < N; i++) (*this)(d[i], s[i]);
+   }
+};
+template <typename R>
+__device__ __forceinline__ void load_hot(HotPlan<R>& h, PlanPtr P)
+{
+   const HotLoad keep;
+   const spx_plan_desc* g = (const spx_plan_desc*)P;   // the compiler follows the address space through the cast
+#define SPX_HOT(m) keep(h.m, g->m)
+   SPX_HOT(traj_type); SPX_HOT(n_bnd); SPX_HOT(n_bt); SPX_HOT(max_steps); SPX_HOT(dt_scale); SPX_HOT(src_p_inj); SPX_HOT(src_rate);
+#undef SPX_HOT
+   const spx_bg_t<R>& b = hot_bg(g, (R*)nullptr);
+#define SPX_HOT(m) keep(h.vbg.m, b.m)
+   SPX_HOT(kind); SPX_HOT(ep_diag); SPX_HOT(t0); SPX_HOT(r0); SPX_HOT(u0); SPX_HOT(B0); SPX_HOT(dmax0); SPX_HOT(r_ref); SPX_HOT(dmax_fraction);
+   SPX_HOT(eprime[0]); SPX_HOT(eprime[1]); SPX_HOT(eprime[2]); SPX_HOT(ur0); SPX_HOT(w0); SPX_HOT(hp_rad); SPX_HOT(ur0_rcp); SPX_HOT(sw_c1);
+   SPX_HOT(sw_k); SPX_HOT(sw_kg); SPX_HOT(sw_r2_ok); SPX_HOT(n_shock); SPX_HOT(v_shock); SPX_HOT(compression); SPX_HOT(u1); SPX_HOT(B1);
+   SPX_HOT(E0); SPX_HOT(E1); SPX_HOT(width_shock); SPX_HOT(Eu);
+   SPX_HOT(grid.nb); SPX_HOT(grid.nz); SPX_HOT(grid.dom_min); SPX_HOT(grid.dom_max); SPX_HOT(grid.block_length); SPX_HOT(grid.f_len);
+   SPX_HOT(grid.f_vel); SPX_HOT(grid.f_mag); SPX_HOT(grid.bmag_min); SPX_HOT(grid.inner_lo); SPX_HOT(grid.inner_hi); SPX_HOT(grid.fd_fields);
+   SPX_HOT(grid.z64); SPX_HOT(grid.c32);
+#undef SPX_HOT
+   const spx_df_t<R>& f = hot_df(g, (R*)nullptr);
+#define SPX_HOT(m) keep(h.vdf.m, f.m)
+   SPX_HOT(kind); SPX_HOT(stream_dep_idx); SPX_HOT(pos_dep); SPX_HOT(region_idx); SPX_HOT(D0); SPX_HOT(Dperp); SPX_HOT(Dpara); SPX_HOT(kap0);
+   SPX_HOT(U0); SPX_HOT(pow_law_U); SPX_HOT(p0); SPX_HOT(pow_law_p); SPX_HOT(kap_rat); SPX_HOT(T0); SPX_HOT(r0); SPX_HOT(pow_law_T);
+   SPX_HOT(pow_law_r); SPX_HOT(u_up); SPX_HOT(w_sh); SPX_HOT(s_sh); SPX_HOT(dn_up_rat); SPX_HOT(lam0); SPX_HOT(R0); SPX_HOT(B0);
+   SPX_HOT(pow_law_R); SPX_HOT(pow_law_B); SPX_HOT(lam_in); SPX_HOT(lam_out); SPX_HOT(kap_rat_in); SPX_HOT(kap_rat_out); SPX_HOT(A2A);
+   SPX_HOT(k_min); SPX_HOT(ps_minus); SPX_HOT(A2T); SPX_HOT(A2L); SPX_HOT(ps_plus); SPX_HOT(l_max_HP); SPX_HOT(z_nose); SPX_HOT(z_sheath);
+   SPX_HOT(k_min_ref); SPX_HOT(A2A_ref); SPX_HOT(A2T_ref); SPX_HOT(A2L_ref); SPX_HOT(dl_max); SPX_HOT(dz); SPX_HOT(hyp_c); SPX_HOT(hyp_g);
+   SPX_HOT(hyp_r); SPX_HOT(lam_para); SPX_HOT(lam_perp); SPX_HOT(kap_rat_red); SPX_HOT(r_lim_red); SPX_HOT(sc_den);
+#undef SPX_HOT
+#pragma unroll
+   for (int k = 0; k < SPX_MAX_BND; k++) {
+#define SPX_HOT(m) keep(h.bnd[k].m, g->bnd[k].m)
+      SPX_HOT(cls); SPX_HOT(kind); SPX_HOT(status0); SPX_HOT(max_crossings); SPX_HOT(same_origin); SPX_HOT(timemark); SPX_HOT(origin);
+      SPX_HOT(radius); SPX_HOT(norm); SPX_HOT(momentum);
+#undef SPX_HOT
+   }
+}
+
 template <typename R> __device__ v3<R> v3of(const SPX_CP R* a) { return mk<R>(a[0], a[1], a[2]); }
+template <typename R> __device__ v3<R> v3of(const R* a) { return mk<R>(a[0], a[1], a[2]); }
 
 // Relative position x - r0 (double subtraction, then the step type).
-template <typename R>
-SPX_HD v3<R> rel(const SPX_CP spx_bg_t<R>& b, double x, double y, double z) { return mk<R>(R(x - b.r0[0]), R(y - b.r0[1]), R(z - b.r0[2])); }
+template <typename BD, typename R = typename BD::real>
+SPX_HD v3<R> rel(BD& b, double x, double y, double z) { return mk<R>(R(x - b.r0[0]), R(y - b.r0[1]), R(z - b.r0[2])); }
 
 // BackgroundSolarWind::EvaluateBackground (src/background_solarwind.cc:111-255), every switch at 0, in
 // the frame of the rotation axis: pp is the position in that frame, u and Bl the fields in it.
-template <typename R>
-SPX_HD void solarwind_local(const SPX_CP spx_bg_t<R>& b, v3<R> pp, int want, v3<R>& u, v3<R>& Bl)
+template <typename R, typename BD>
+SPX_HD void solarwind_local(BD& b, v3<R> pp, int want, v3<R>& u, v3<R>& Bl)
 {
    if constexpr (is_f32<R>()) {
       // The spiral in closed form: sin(theta) cos(phi) = x / r, sin(theta) sin(phi) = y / r, cos(theta) = z / r,
@@ -185,8 +263,8 @@ SPX_HD void solarwind_local(const SPX_CP spx_bg_t<R>& b, v3<R> pp, int want, v3<
 // from_basis reduce to sign flips: every product with an off-diagonal zero adds a signed zero, so the
 // results agree bit for bit up to the sign of a zero.  The identity basis (rotation axis along +z,
 // a uniform branch) needs no products at all: x * 1 == x exactly.
-template <typename R>
-SPX_HD void solarwind_eval(const SPX_CP spx_bg_t<R>& b, v3<R> d, int want, v3<R>& U, v3<R>& B)
+template <typename R, typename BD>
+SPX_HD void solarwind_eval(BD& b, v3<R> d, int want, v3<R>& U, v3<R>& B)
 {
    if (is_f32<R>() && b.ep_diag != 0) {
       // the closed form in the global frame: a diagonal basis S (det 1) turns S w(S d) into
@@ -221,8 +299,8 @@ SPX_HD void solarwind_eval(const SPX_CP spx_bg_t<R>& b, v3<R> d, int want, v3<R>
 //
 // NumericalDerivatives' trace for div U (src/background_base.cc:228-312 with the basis e_k):
 // sum_k e_k . [U(c + h e_k) - U(c - h e_k)], with e . U(p) = ur0 (e . p) / |p|.
-template <typename R>
-SPX_HD R sw_divu_stencil(const SPX_CP spx_bg_t<R>& b, v3<R> c, R h, const v3<R> (&e)[3])
+template <typename R, typename BD>
+SPX_HD R sw_divu_stencil(BD& b, v3<R> c, R h, const v3<R> (&e)[3])
 {
    const R c2h = norm2(c) + h * h, h2 = R(2) * h;
    R acc = R(0);
@@ -240,14 +318,14 @@ SPX_HD R sw_divu_stencil(const SPX_CP spx_bg_t<R>& b, v3<R> c, R h, const v3<R> 
 // in b_j b = w_j w / |w|^2.
 // True when no point c +- h e_j can meet GetFields' |B| < sp_tiny (src/background_base.cc:444-448): every
 // |c +- h e_j|^2 is at most |c|^2 + h^2 + 2h (|c_x| + |c_y| + |c_z|).
-template <typename R>
-SPX_HD bool sw_stencil_clear(const SPX_CP spx_bg_t<R>& b, v3<R> c, R h)
+template <typename R, typename BD>
+SPX_HD bool sw_stencil_clear(BD& b, v3<R> c, R h)
 {
    return norm2(c) + h * h + (R(2) * h) * (fabs(c.x) + fabs(c.y) + fabs(c.z)) <= b.sw_r2_ok;
 }
 
-template <typename R>
-SPX_HD v3<R> sw_bb_stencil(const SPX_CP spx_bg_t<R>& b, v3<R> c, R h)
+template <typename R, typename BD>
+SPX_HD v3<R> sw_bb_stencil(BD& b, v3<R> c, R h)
 {
    const R c2h = norm2(c) + h * h, h2 = R(2) * h;
    v3<R> acc = mk<R>(R(0), R(0), R(0));
@@ -276,8 +354,8 @@ template <typename R> SPX_HD R shock_transition_deriv(R x) { return R(0.5) * R(8
 
 // Generic EvaluateBackground for U and B (want bits) at d = x - r0, used at the finite-difference
 // points.  `ds` receives BackgroundSmoothShock's transition coordinate of this evaluation.
-template <typename R, int BG>
-SPX_HD void bg_eval_rel(const SPX_CP spx_bg_t<R>& b, double t, v3<R> d, int want, v3<R>& U, v3<R>& B, R& ds)
+template <typename R, int BG, typename BD>
+SPX_HD void bg_eval_rel(BD& b, double t, v3<R> d, int want, v3<R>& U, v3<R>& B, R& ds)
 {
    if (BG == SPX_BG_SOLARWIND) {
       solarwind_eval<R>(b, d, want, U, B);
@@ -297,16 +375,16 @@ SPX_HD void bg_eval_rel(const SPX_CP spx_bg_t<R>& b, double t, v3<R> d, int want
    }
 }
 
-template <typename R, int BG>
-SPX_HD void bg_eval(const SPX_CP spx_bg_t<R>& b, double t, double x, double y, double z, int want, v3<R>& U, v3<R>& B, R& ds)
+template <typename R, int BG, typename BD>
+SPX_HD void bg_eval(BD& b, double t, double x, double y, double z, int want, v3<R>& U, v3<R>& B, R& ds)
 {
    bg_eval_rel<R, BG>(b, t, rel(b, x, y, z), want, U, B, ds);
 }
 
 // EvaluateDmax per class (src/background_solarwind.cc:310-314, src/background_smooth_shock.cc:192-196,
 // src/background_base.cc:378-382).  `ds_prev` is the smooth shock coordinate of the previous evaluation.
-template <typename R, int BG>
-SPX_HD R bg_dmax(const SPX_CP spx_bg_t<R>& b, double x, double y, double z, R ds_prev)
+template <typename R, int BG, typename BD>
+SPX_HD R bg_dmax(BD& b, double x, double y, double z, R ds_prev)
 {
    if (BG == SPX_BG_SOLARWIND) return fmin(b.dmax_fraction * norm(rel(b, x, y, z)), b.dmax0);
    if (BG == SPX_BG_SMOOTHSHOCK) return fmin(b.dmax_fraction * b.width_shock * fmax(R(1), fabs(ds_prev)), b.dmax0);
@@ -338,25 +416,26 @@ typedef float grid_f4 __attribute__((ext_vector_type(4)));
 
 // Corner c = i + 2j + 4k of the stencil whose lowest zone is `cell`: that zone record (U, B, |B|, fluid
 // units).  FP64 reads it from the zone array, FP32 from the cell's contiguous copy of its 8 corners.
-template <typename R> __device__ __forceinline__ void grid_corner(const SPX_CP spx_grid_desc& g, int64_t cell, int c, R v[7]);
-template <> __device__ __forceinline__ void grid_corner<double>(const SPX_CP spx_grid_desc& g, int64_t cell, int c, double v[7])
+template <typename R, typename GD>
+__device__ __forceinline__ void grid_corner(GD& g, int64_t cell, int c, R v[7])
 {
-   const int64_t zone = cell + (c & 1) + ((c >> 1) & 1) * (int64_t)g.nz[0] + (c >> 2) * ((int64_t)g.nz[0] * g.nz[1]);
-   const grid_d2* r = reinterpret_cast<const grid_d2*>(g.z64) + zone * (SPX_GRID_REC / 2);
-   const grid_d2 a = r[0], b = r[1], d = r[2], e = r[3];
-   v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y; v[4] = d.x; v[5] = d.y; v[6] = e.x;
-}
-template <> __device__ __forceinline__ void grid_corner<float>(const SPX_CP spx_grid_desc& g, int64_t cell, int c, float v[7])
-{
-   const grid_f4* r = reinterpret_cast<const grid_f4*>(g.c32) + (cell * 8 + c) * (SPX_GRID_REC / 4);
-   const grid_f4 a = r[0], b = r[1];
-   v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z;
+   if constexpr (is_f32<R>()) {
+      const grid_f4* r = reinterpret_cast<const grid_f4*>(g.c32) + (cell * 8 + c) * (SPX_GRID_REC / 4);
+      const grid_f4 a = r[0], b = r[1];
+      v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z;
+   }
+   else {
+      const int64_t zone = cell + (c & 1) + ((c >> 1) & 1) * (int64_t)g.nz[0] + (c >> 2) * ((int64_t)g.nz[0] * g.nz[1]);
+      const grid_d2* r = reinterpret_cast<const grid_d2*>(g.z64) + zone * (SPX_GRID_REC / 2);
+      const grid_d2 a = r[0], b = r[1], d = r[2], e = r[3];
+      v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y; v[4] = d.x; v[5] = d.y; v[6] = e.x;
+   }
 }
 
 // The position's block, its stencil's first zone and the offsets within it.  False where the
 // reference fails (outside the domain, or a stencil beyond the grid).
-template <typename R>
-__device__ __forceinline__ bool grid_locate(const SPX_CP spx_grid_desc& g, double x, double y, double z, R lo[3], R hi[3], R dl[3],
+template <typename R, typename GD>
+__device__ __forceinline__ bool grid_locate(GD& g, double x, double y, double z, R lo[3], R hi[3], R dl[3],
                                             int64_t& zone0, double& zl_min)
 {
    const double pos[3] = {x, y, z};
@@ -387,8 +466,8 @@ __device__ __forceinline__ bool grid_locate(const SPX_CP spx_grid_desc& g, doubl
    return true;
 }
 
-template <typename R>
-__device__ __forceinline__ bool grid_inside(const SPX_CP spx_grid_desc& g, double x, double y, double z)
+template <typename R, typename GD>
+__device__ __forceinline__ bool grid_inside(GD& g, double x, double y, double z)
 {
    // well inside the zone-centre box the answer is yes without the exact block arithmetic
    if (x > g.inner_lo[0] && x < g.inner_hi[0] && y > g.inner_lo[1] && y < g.inner_hi[1] && z > g.inner_lo[2] && z < g.inner_hi[2])
@@ -399,8 +478,8 @@ __device__ __forceinline__ bool grid_inside(const SPX_CP spx_grid_desc& g, doubl
    return grid_locate<R>(g, x, y, z, lo, hi, dl, zone0, zl_min);
 }
 
-template <typename R, bool GRAD>
-__device__ __forceinline__ bool grid_eval(const SPX_CP spx_grid_desc& g, double x, double y, double z, GridFields<R>& o)
+template <typename R, bool GRAD, typename GD>
+__device__ __forceinline__ bool grid_eval(GD& g, double x, double y, double z, GridFields<R>& o)
 {
    R lo[3], hi[3], dl[3];
    int64_t zone0;
@@ -448,8 +527,8 @@ __device__ __forceinline__ bool grid_eval(const SPX_CP spx_grid_desc& g, double 
 // units before the unit conversion (GetVariablesInterp1, src/server_cartesian.cc:538-560, :590-609), and
 // from the stencil's derivative weights (GetGradientsInterp1, :630-705) grad|B| and the off-diagonal
 // d B_j / d x_i that curl B needs.  gB holds (01, 02, 10, 12, 20, 21) of gradB[i][j] = d B_j / d x_i.
-template <typename R>
-__device__ __forceinline__ bool grid_eval_gc(const SPX_CP spx_grid_desc& g, double x, double y, double z, v3<R>& U, v3<R>& B, R& Bmag,
+template <typename R, typename GD>
+__device__ __forceinline__ bool grid_eval_gc(GD& g, double x, double y, double z, v3<R>& U, v3<R>& B, R& Bmag,
                                              v3<R>& E, v3<R>& gradBmag, R gB[6], double& zl_min)
 {
    R lo[3], hi[3], dl[3];
@@ -504,8 +583,8 @@ __device__ __forceinline__ bool grid_eval_gc(const SPX_CP spx_grid_desc& g, doub
 // focused transport (GRADS = true: also grad U and grad B row by row, gU[i] = d U / d x_i, and grad |B|),
 // from the stencil's weights and derivative weights (GetVariablesInterp1 / GetGradientsInterp1,
 // src/server_cartesian.cc:538-609, :630-705); E = -(U x B) / c in fluid units before the unit conversion.
-template <typename R, bool GRADS>
-__device__ __forceinline__ bool grid_eval_full(const SPX_CP spx_grid_desc& g, double x, double y, double z, v3<R>& U, v3<R>& B, R& Bmag,
+template <typename R, bool GRADS, typename GD>
+__device__ __forceinline__ bool grid_eval_full(GD& g, double x, double y, double z, v3<R>& U, v3<R>& B, R& Bmag,
                                                v3<R>& E, v3<R> (&gU)[3], v3<R> (&gB)[3], v3<R>& gradBmag, double& zl_min)
 {
    R lo[3], hi[3], dl[3];
@@ -572,8 +651,8 @@ SPX_HD float rcbrt(float x) { return cbrtf(x); }
 // DiffusionStraussEtAl2013 (src/diffusion_other.cc:886-906) and DiffusionPotgieterEtAl2015 (:968-988):
 // kappa_par = (lam v / 3) f(R) (B0_eff / |B|), resp. kappa (v / c) g(R) (B0_eff / |B|); this is the factor
 // before (B0_eff / |B|) for the inner (heliosphere) or outer (LISM) parameters, in the reference's order.
-template <typename R>
-SPX_HD R kappa_mom_region(const SPX_CP spx_df_t<R>& d, R p, bool outer)
+template <typename R, typename DD>
+SPX_HD R kappa_mom_region(DD& d, R p, bool outer)
 {
    const R lam = outer ? d.lam_out : d.lam_in;
    const R rig = Rigidity(p), vmag = VelP(p);
@@ -586,8 +665,8 @@ SPX_HD R kappa_mom_region(const SPX_CP spx_df_t<R>& d, R p, bool outer)
 // with the bent power laws f = cbrt(x (1 + x^4)) (parallel), cbrt(x (1 + x^2)) (perpendicular), x = R / R0.
 // This is the factor before (B0 / |B|), for the parallel component or for the perpendicular one with the
 // mean free path lam_perp (reduced = false) or lam_perp kap_rat_red (reduced = true), in the reference's order.
-template <typename R>
-SPX_HD R kappa_mom_soqlt(const SPX_CP spx_df_t<R>& d, R p, int comp, bool reduced)
+template <typename R, typename DD>
+SPX_HD R kappa_mom_soqlt(DD& d, R p, int comp, bool reduced)
 {
    const R rig = Rigidity(p), vmag = VelP(p);
    const R x = rig / d.R0;
@@ -599,8 +678,8 @@ SPX_HD R kappa_mom_soqlt(const SPX_CP spx_df_t<R>& d, R p, int comp, bool reduce
 
 // The momentum-only factor of kappa_par: the same at every point of a step's derivative stencil, so
 // it is formed once per step (the same inputs give the same value).
-template <typename R>
-SPX_HD R kappa_mom(const SPX_CP spx_df_t<R>& d, R p)
+template <typename R, typename DD>
+SPX_HD R kappa_mom(DD& d, R p)
 {
    switch (d.kind) {
    case SPX_DF_FLOWMOM: return rpow(p / d.p0, d.pow_law_p);                                   // :622-627
@@ -614,8 +693,8 @@ SPX_HD R kappa_mom(const SPX_CP spx_df_t<R>& d, R p)
 
 // Kappa components 0 (perp) and 1 (para) at one point, in the reference's operation order; km is
 // kappa_mom, r is |x| (KINRAD), Umag |U|.
-template <typename R>
-SPX_HD void kappa01(const SPX_CP spx_df_t<R>& d, R km, R Bmag, R r, R Umag, R& K0, R& K1)
+template <typename R, typename DD>
+SPX_HD void kappa01(DD& d, R km, R Bmag, R r, R Umag, R& K0, R& K1)
 {
    switch (d.kind) {
    case SPX_DF_PARA: K1 = d.D0; break;                                      // :381-385

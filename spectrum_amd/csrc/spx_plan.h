@@ -61,6 +61,7 @@ typedef struct {
 // Background parameters in the step type T (double for the drop-in kernel, float for the mixed one).
 template <typename T>
 struct spx_bg_t {
+   typedef T real;
    int32_t kind;
    int32_t ep_diag;                    // SolarWind: eprime is diagonal with entries +-1 (rotation axis along +-z); 2: the identity
    double t0, r0[3];                   // always double: positions are accumulated in double

@@ -129,6 +129,15 @@ void QueryRes::release()
    std::memset(&desc, 0, sizeof(desc));
 }
 
+uint64_t few_limit()
+{
+   static const uint64_t lanes = [] {
+      hipDeviceProp_t prop;
+      return hipGetDeviceProperties(&prop, 0) == hipSuccess ? (uint64_t)prop.multiProcessorCount * 4 * 64 / 4 : (uint64_t)0;
+   }();
+   return lanes;
+}
+
 // ---- Pool -------------------------------------------------------------------------------------
 bool Pool::matches(const spx_plan_desc& p, int prec) const
 {
@@ -222,8 +231,11 @@ hipError_t Pool::set_query(int q, const QueryDesc& d)
    return hipStreamSynchronize(stream);
 }
 
-hipError_t Pool::push_queue(int q)
+hipError_t Pool::push_queue(int q, uint64_t n_traj)
 {
+   if (host_queue.empty()) span = 0;   // every slot is idle
+   const uint64_t want = n_traj < n_lanes ? (n_traj + 255) / 256 * 256 : n_lanes;
+   span = std::min(n_lanes, span + want);
    host_queue.push_back(q);
    return upload_launch();
 }
@@ -234,13 +246,13 @@ hipError_t Pool::remove_queue(int q)
    return upload_launch();
 }
 
-hipError_t Pool::enqueue(int n)
+hipError_t Pool::enqueue(int n, uint64_t live)
 {
    if (graph_launches > 0) {
       if (!graph_exec) {
          TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
          for (int i = 0; i < graph_launches; i++) {
-            hipError_t e = launch_transport(sig, n_lanes, d_launch.p, precision, stream, nullptr);
+            hipError_t e = launch_transport(sig, n_lanes, d_launch.p, precision, false, stream, nullptr);
             if (e != hipSuccess) {
                hipGraph_t g;
                (void)hipStreamEndCapture(stream, &g);
@@ -255,16 +267,16 @@ hipError_t Pool::enqueue(int n)
       launches += (int64_t)reps * graph_launches;
       return hipSuccess;
    }
-   for (int i = 0; i < n; i++) TRY(launch_transport(sig, n_lanes, d_launch.p, precision, stream, nullptr));
+   for (int i = 0; i < n; i++) TRY(launch_transport(sig, span, d_launch.p, precision, few(live), stream, nullptr));
    launches += n;
    return hipSuccess;
 }
 
-hipError_t Pool::launch(int n, float* ms_out)
+hipError_t Pool::launch(int n, uint64_t live, float* ms_out)
 {
    TRY(hipEventRecord(ev0, stream));
    if (graph_launches > 0) {
-      TRY(enqueue(n));
+      TRY(enqueue(n, live));
    }
    else {
       while (tev.size() < (size_t)2 * n) {
@@ -274,7 +286,7 @@ hipError_t Pool::launch(int n, float* ms_out)
       }
       for (int i = 0; i < n; i++) {
          TRY(hipEventRecord(tev[2 * i], stream));
-         TRY(launch_transport(sig, n_lanes, d_launch.p, precision, stream, tev[2 * i + 1]));
+         TRY(launch_transport(sig, span, d_launch.p, precision, few(live), stream, tev[2 * i + 1]));
       }
       launches += n;
    }

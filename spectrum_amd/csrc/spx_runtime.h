@@ -9,6 +9,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <string>
 #include <vector>
 
@@ -67,11 +68,15 @@ int64_t acc_components(const spx_plan_desc& plan);
 hipError_t read_hist(const spx_plan_desc& p, int d, const unsigned long long* dev_counts, const unsigned long long* dev_acc,
                      const unsigned long long* dev_events, int64_t* counts, double* sums, int64_t* n_events, hipStream_t st);
 
+// Trajectories up to which the few-wave step kernels run: their quads fill one wave on every SIMD of the device.
+uint64_t few_limit();
+
 // Resident slots running one kernel instantiation.
 struct Pool {
    spx_plan_desc sig{};                 // host plan whose kinds select the kernels
    int precision = SPX_PREC_FP64;
    uint64_t n_lanes = 0;
+   uint64_t span = 0;                   // slots that may hold a trajectory (whole blocks)
    int steps_per_launch = 2000;
    int graph_launches = 0;
    int qcap = 0;                        // size of the query table
@@ -103,16 +108,19 @@ struct Pool {
    int alloc_index();                   // free query-table entry, or -1
    void free_index(int q);
    hipError_t set_query(int q, const QueryDesc& d);
-   hipError_t push_queue(int q);
+   hipError_t push_queue(int q, uint64_t n_traj);
    hipError_t remove_queue(int q);
-   // enqueue n engine launches on the pool's stream (graph replays when graph_launches > 0)
-   hipError_t enqueue(int n);
+   // enqueue n engine launches on the pool's stream (graph replays when graph_launches > 0); `live` bounds the
+   // trajectories that are running or still to be claimed, and picks the step kernel's form.  The kernels cover
+   // the first `span` slots only: as many as the queries admitted since the pool was last empty can fill.
+   hipError_t enqueue(int n, uint64_t live);
    // enqueue, wait, and account kernel time (ms of the call, step / service kernel split)
-   hipError_t launch(int n, float* ms);
+   hipError_t launch(int n, uint64_t live, float* ms);
    void release();
 
 private:
    hipError_t upload_launch();
+   bool few(uint64_t live) const { return has_few(sig, precision) && std::max(live, span) <= few_limit(); }
 };
 
 }  // namespace spx
