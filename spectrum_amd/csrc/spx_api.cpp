@@ -186,6 +186,7 @@ struct spx_sim {
    uint64_t run_first = 0, run_n = 0;
    bool keep_records = false;
    uint64_t run_done = 0;              // trajectories finished when the control block was last read
+   bool run_claimed = false;           // and whether all had been handed out
    // SimulationMaster's tasks (src/simulation.hh:196-237): trajectory count, batch size, per-worker
    // maximum, the base name of the distribution files, the distributions to restore at the start
    int64_t task_n = 0, task_batch = 0, task_max_per_worker = 0;
@@ -874,6 +875,7 @@ int spx_begin(spx_sim* s, uint64_t first, uint64_t n_traj, const spx_rng* rng, i
    s->run_first = first;
    s->run_n = n_traj;
    s->run_done = 0;
+   s->run_claimed = false;
    s->running = true;
    return SPX_OK;
 }
@@ -883,6 +885,7 @@ static int read_stats(spx_sim* s, spx_run_stats* st, double wall, double kms, in
    RunCtl ctl;
    HIPCHK(s, s->q.read_ctl(ctl, s->pool.stream));
    s->run_done = ctl.done;
+   s->run_claimed = ctl.next >= s->run_first + s->run_n;
    if (st) {
       std::memset(st, 0, sizeof(*st));
       st->n_traj = s->run_n;
@@ -912,7 +915,7 @@ int spx_advance(spx_sim* s, int n_launches, spx_run_stats* st)
    auto w0 = std::chrono::steady_clock::now();
    s->pool.step_ms = s->pool.service_ms = 0.0;
    float ms = 0.f;
-   HIPCHK(s, s->pool.launch(n_launches, s->run_n - std::min(s->run_done, s->run_n), &ms));
+   HIPCHK(s, s->pool.launch(n_launches, s->pool.shape(s->run_n - std::min(s->run_done, s->run_n), s->run_claimed, s->steps_per_launch), &ms));
    double wall = std::chrono::duration<double>(std::chrono::steady_clock::now() - w0).count();
    return read_stats(s, st, wall, ms, n_launches);
 }
@@ -925,21 +928,16 @@ int spx_finish(spx_sim* s, spx_traj_record* records, spx_run_stats* st)
    s->pool.step_ms = s->pool.service_ms = 0.0;
    double kms = 0.0;
    int launches = 0;
-   // Every launch advances each live slot by steps_per_launch steps; a trajectory needs at most
-   // max_attempts * (max_steps + 1) steps, so this bound is never reached by a healthy run.
-   const double guard = 64.0 + (double)s->plan.max_attempts * ((double)s->plan.max_steps + 1.0) / s->steps_per_launch *
+   // Every launch advances each live slot by min(steps_per_launch, 100) steps or more (Pool::round); a trajectory
+   // needs at most max_attempts * (max_steps + 1) steps, so this bound is never reached by a healthy run.
+   const double guard = 64.0 + (double)s->plan.max_attempts * ((double)s->plan.max_steps + 1.0) / std::min(s->steps_per_launch, 100) *
                                    std::max(1.0, (double)s->run_n / (double)s->pool.n_lanes + 1.0);
-   int batch = 1;
    while (true) {
       RunCtl ctl;
       HIPCHK(s, s->q.read_ctl(ctl, s->pool.stream));
       if (ctl.done >= s->run_n) break;
       if (launches > guard) return fail(s, SPX_ERR_STATE, "run did not drain");
-      float ms = 0.f;
-      HIPCHK(s, s->pool.launch(batch, s->run_n - ctl.done, &ms));
-      kms += ms;
-      launches += batch;
-      if (batch < 8) batch *= 2;
+      HIPCHK(s, s->pool.round(s->run_n - ctl.done, ctl.next >= s->run_first + s->run_n, kms, launches));
    }
    double wall = std::chrono::duration<double>(std::chrono::steady_clock::now() - w0).count();
    int rc = read_stats(s, st, wall, kms, launches);
@@ -1378,9 +1376,9 @@ int spx_main_loop(spx_sim* s, const spx_rng* rng, spx_run_stats* st)
       if (rc) return rc;
       const auto w0 = std::chrono::steady_clock::now();
       s->pool.step_ms = s->pool.service_ms = 0.0;
-      const double guard = 64.0 + (double)s->plan.max_attempts * ((double)s->plan.max_steps + 1.0) / s->steps_per_launch *
+      const double guard = 64.0 + (double)s->plan.max_attempts * ((double)s->plan.max_steps + 1.0) / std::min(s->steps_per_launch, 100) *
                                       std::max(1.0, (double)n_total / (double)s->pool.n_lanes + 1.0);
-      int percentage_done = 0, launches = 0, burst = 1;
+      int percentage_done = 0, launches = 0;
       while (true) {
          RunCtl ctl;
          HIPCHK(s, s->q.read_ctl(ctl, s->pool.stream));
@@ -1407,11 +1405,7 @@ int spx_main_loop(spx_sim* s, const spx_rng* rng, spx_run_stats* st)
          }
          if (done >= n_total) break;
          if (launches > guard) return fail(s, SPX_ERR_STATE, "run did not drain");
-         float ms = 0.f;
-         HIPCHK(s, s->pool.launch(burst, (uint64_t)(n_total - done), &ms));
-         integ_ms += ms;
-         launches += burst;
-         if (burst < 8) burst *= 2;
+         HIPCHK(s, s->pool.round((uint64_t)(n_total - done), ctl.next >= s->run_first + s->run_n, integ_ms, launches));
       }
       const double wall = std::chrono::duration<double>(std::chrono::steady_clock::now() - w0).count();
       rc = spx_finish(s, nullptr, &run);
@@ -1582,9 +1576,13 @@ static void server_loop(spx_server* S)
          for (Pool* pl : S->pools) {
             if (pl->host_queue.empty()) continue;
             uint64_t live = 0;
+            bool claimed = true;
             for (const SQuery* q : S->running)   // this thread alone changes the list and the counters
-               if (q->pool == pl) live += q->n_traj - std::min<uint64_t>(q->ctl.done, q->n_traj);
-            hipError_t e = pl->enqueue(S->o.launches_per_poll, live);
+               if (q->pool == pl) {
+                  live += q->n_traj - std::min<uint64_t>(q->ctl.done, q->n_traj);
+                  claimed = claimed && q->ctl.next >= q->first + q->n_traj;
+               }
+            hipError_t e = pl->enqueue(S->o.launches_per_poll, pl->shape(live, claimed, pl->steps_per_launch));
             if (e != hipSuccess) { server_fail(S, std::string("launch: ") + hipGetErrorString(e)); goto out; }
             any = true;
          }

@@ -101,11 +101,18 @@ template <typename R> __device__ __forceinline__ void own_rounding1(v3<R>& v)
 // this it would fuse the multiply of the term already in the sum instead of the next one's, as the loop does.
 template <typename... T> __device__ __forceinline__ void own_rounding(T&... v) { (own_rounding1(v), ...); }
 __device__ __forceinline__ int quad_lane() { return (int)threadIdx.x & (QUAD - 1); }
-// The slot of a lane in a step kernel, and whether the lane writes for it.
-template <int V> __device__ __forceinline__ uint64_t slot_of()
+// The slot of a lane in a step kernel (-1: none), and whether the lane writes for it.  The running slots come from
+// the launch's list when it is packed; a wave whose first place is empty has none.
+template <int V> __device__ __forceinline__ int32_t slot_of(LaunchPtr L, int32_t packed)
 {
-   const uint64_t i = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
-   return V == 1 ? i / QUAD : i;
+   const uint64_t i = ((uint64_t)blockIdx.x * BLOCK + threadIdx.x) / (V == 1 ? QUAD : 1);
+   return packed >= 0 ? L->list[i] : (int32_t)i;
+}
+inline unsigned service_grid(const LaunchShape& S) { return (unsigned)((S.span + BLOCK - 1) / BLOCK); }
+template <int V> inline unsigned step_grid(const LaunchShape& S)
+{
+   const uint64_t n = S.packed >= 0 ? S.list_span : S.span;
+   return (unsigned)((n * (V == 1 ? QUAD : 1) + BLOCK - 1) / BLOCK);
 }
 template <int V> __device__ __forceinline__ bool slot_writer() { return V != 1 || quad_lane() == 0; }
 
@@ -711,7 +718,8 @@ __device__ __forceinline__ int handle_boundaries(PP P, PlanPtr Pc, LaunchPtr L, 
 // ---------------------------------------------------------------------------------------------
 // Service pass, one thread per slot: bin the events the step kernel queued, finish or retry
 // trajectories, refill idle slots from their query's work counter (moving a fully idle wave to the
-// oldest admitted query with trajectories left) and run SetStart through `set_start`, a functor
+// oldest admitted query with trajectories left), run SetStart, and number the running slots of each query for a
+// packed launch.  SetStart runs through `set_start`, a functor
 // (plan, query, rng, slot, traj, nu&) -> exception code of the transport.
 // ---------------------------------------------------------------------------------------------
 __device__ __forceinline__ unsigned long long load_next(const RunCtl* ctl)
@@ -720,7 +728,7 @@ __device__ __forceinline__ unsigned long long load_next(const RunCtl* ctl)
 }
 
 template <typename StartFn>
-__device__ __forceinline__ void service_slot(LaunchPtr L, StartFn&& set_start)
+__device__ __forceinline__ void service_slot(LaunchPtr L, int32_t packed, StartFn&& set_start)
 {
    const uint64_t slot = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
    int st = L->active[slot];
@@ -836,6 +844,16 @@ __device__ __forceinline__ void service_slot(LaunchPtr L, StartFn&& set_start)
       }
    }
    L->active[slot] = st;
+   // 5. for a packed launch: this slot's place among the running slots of its query (one atomic per wave)
+   if (packed >= 0) {
+      const uint64_t mask = __ballot(st == SLOT_RUN);
+      if (mask != 0) {
+         uint32_t base = 0;
+         if (lane_id() == 0) base = atomicAdd(&L->n_running[packed * L->n_queries + q], (uint32_t)__popcll(mask));
+         base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+         if (st == SLOT_RUN) L->rank[slot] = (int32_t)(base + (uint32_t)__popcll(mask & lanes_below()));
+      }
+   }
 }
 
 }  // namespace spx

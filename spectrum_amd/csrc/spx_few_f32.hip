@@ -9,11 +9,11 @@
 
 namespace spx {
 
-hipError_t launch_few_f32(const spx_plan_desc& hp, uint64_t n_lanes, const Launch* d_launch, hipStream_t st)
+hipError_t launch_few_f32(const spx_plan_desc& hp, const LaunchShape& S, const Launch* d_launch, hipStream_t st)
 {
    switch (hp.bg.kind) {
-   case SPX_BG_GRID: return dispatch_grid<float, LAUNCH_FEW>(hp, n_lanes, d_launch, st, nullptr);
-   case SPX_BG_SOLARWIND: return dispatch_flow<float, SPX_BG_SOLARWIND, LAUNCH_FEW>(hp, n_lanes, d_launch, st, nullptr);
+   case SPX_BG_GRID: return dispatch_grid<float, LAUNCH_FEW>(hp, S, d_launch, st, nullptr);
+   case SPX_BG_SOLARWIND: return dispatch_flow<float, SPX_BG_SOLARWIND, LAUNCH_FEW>(hp, S, d_launch, st, nullptr);
    default: return hipErrorInvalidValue;
    }
 }

@@ -6,11 +6,11 @@
 
 namespace spx {
 
-hipError_t launch_few_f64(const spx_plan_desc& hp, uint64_t n_lanes, const Launch* d_launch, hipStream_t st)
+hipError_t launch_few_f64(const spx_plan_desc& hp, const LaunchShape& S, const Launch* d_launch, hipStream_t st)
 {
    if (hp.traj_type >= SPX_TRAJ_GUIDING_DIFF_SCATT && hp.traj_type <= SPX_TRAJ_GUIDING_DIFF)
-      return dispatch_gc<double, LAUNCH_FEW>(hp, n_lanes, d_launch, st, nullptr);
-   return dispatch_parker<double, LAUNCH_FEW>(hp, n_lanes, d_launch, st, nullptr);
+      return dispatch_gc<double, LAUNCH_FEW>(hp, S, d_launch, st, nullptr);
+   return dispatch_parker<double, LAUNCH_FEW>(hp, S, d_launch, st, nullptr);
 }
 
 }  // namespace spx

@@ -428,10 +428,10 @@ __device__ int gc_set_start(PlanPtr P, QueryPtr Q, LaunchPtr L, const spx_rng_de
 }
 
 template <typename R, int BG>
-__global__ __launch_bounds__(BLOCK) void gc_service(const Launch* __restrict__ Lg)
+__global__ __launch_bounds__(BLOCK) void gc_service(const Launch* __restrict__ Lg, int32_t packed)
 {
    const LaunchPtr L = (LaunchPtr)Lg;
-   service_slot(L, [&](PlanPtr P, QueryPtr Q, const spx_rng_desc& rng, uint64_t slot, uint64_t traj, uint32_t& nu) {
+   service_slot(L, packed, [&](PlanPtr P, QueryPtr Q, const spx_rng_desc& rng, uint64_t slot, uint64_t traj, uint32_t& nu) {
       return gc_set_start<R, BG>(P, Q, L, rng, slot, traj, nu);
    });
 }
@@ -602,17 +602,20 @@ __device__ __forceinline__ int gc_step(PP P, PlanPtr Pc, LaunchPtr L, const spx_
 #endif
 
 template <typename R, int BG, bool XD, int V>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(V == 1 ? 1 : SPX_GC_WAVES))) void gc_step_kernel(const Launch* __restrict__ Lg)
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(V == 1 ? 1 : SPX_GC_WAVES))) void gc_step_kernel(const Launch* __restrict__ Lg, int32_t packed, int32_t n_steps)
 {
    const LaunchPtr Lp = (LaunchPtr)Lg;
    __shared__ ColdLDS C;
    const int tid = threadIdx.x;
    __shared__ RingLDS<R, V> ring;
-   const uint64_t slot = slot_of<V>();
+   const int32_t place = slot_of<V>(Lp, packed);
+   const int32_t place0 = __builtin_amdgcn_readfirstlane(place);
+   if (place0 < 0) return;
+   const uint64_t slot = place < 0 ? (uint64_t)place0 : (uint64_t)place;
    const bool writer = slot_writer<V>();
    // the slots of a wave work for one query (the pool size is a multiple of the block size)
    const int q = __builtin_amdgcn_readfirstlane(Lp->slot_q[slot]);
-   const bool run = q >= 0 && Lp->active[slot] == SLOT_RUN;
+   const bool run = q >= 0 && place >= 0 && Lp->active[slot] == SLOT_RUN;
    if (__ballot(run) == 0) return;
    const QueryPtr Q = query_of(Lp, q);
    const PlanPtr P = plan_of(Q);
@@ -649,7 +652,6 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(V == 1 ? 
    unsigned long long steps_here = 0;
    HotPlan<R> hot;
    if constexpr (V == 1 && !is_f32<R>()) load_hot(hot, P);
-   const int n_steps = Lp->steps_per_launch;
    for (int it = 0; it < n_steps; it++) {
       if (__ballot(st == SLOT_RUN) == 0) break;
       if (st != SLOT_RUN) continue;
@@ -696,24 +698,27 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(V == 1 ? 
 }
 
 template <typename R, int BG, bool XD, int M>
-static hipError_t launch_gc_bg(uint64_t n_lanes, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
+static hipError_t launch_gc_bg(const LaunchShape& S, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
 {
-   const unsigned grid = (unsigned)((n_lanes + BLOCK - 1) / BLOCK);   // n_lanes: the slots that may hold a trajectory
    if constexpr (M != LAUNCH_FEW) {
-      hipLaunchKernelGGL((gc_service<R, BG>), dim3(grid), dim3(BLOCK), 0, st, d_launch);
+      hipLaunchKernelGGL((gc_service<R, BG>), dim3(service_grid(S)), dim3(BLOCK), 0, st, d_launch, S.packed);
+      if (S.packed >= 0) {
+         hipError_t e = pack_running(S, d_launch, st);
+         if (e != hipSuccess) return e;
+      }
       if (mid) {
          hipError_t e = hipEventRecord(mid, st);
          if (e != hipSuccess) return e;
       }
    }
+   constexpr int V = (M == LAUNCH_FEW) ? 1 : 0;
    if constexpr (M != LAUNCH_SERVICE)
-      hipLaunchKernelGGL((gc_step_kernel<R, BG, XD, (M == LAUNCH_FEW ? 1 : 0)>), dim3(M == LAUNCH_FEW ? grid * QUAD : grid), dim3(BLOCK), 0, st,
-                         d_launch);
+      hipLaunchKernelGGL((gc_step_kernel<R, BG, XD, V>), dim3(step_grid<V>(S)), dim3(BLOCK), 0, st, d_launch, S.packed, S.n_steps);
    return hipGetLastError();
 }
 
 template <typename R, int M>
-hipError_t dispatch_gc(const spx_plan_desc& hp, uint64_t n_lanes, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
+hipError_t dispatch_gc(const spx_plan_desc& hp, const LaunchShape& S, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
 {
    if (hp.time_flow != 0) return hipErrorInvalidValue;
    // the WNLT, Strauss / Potgieter and SOQLT models run in kernels of their own (SolarWind, Uniform)
@@ -721,12 +726,12 @@ hipError_t dispatch_gc(const spx_plan_desc& hp, uint64_t n_lanes, const Launch* 
    const bool xd = (k == SPX_DF_WNLT || k == SPX_DF_WNLT_RAMP || k == SPX_DF_STRAUSS || k == SPX_DF_POTGIETER || k == SPX_DF_SOQLT);
    switch (hp.bg.kind) {
    case SPX_BG_SOLARWIND:
-      return xd ? launch_gc_bg<R, SPX_BG_SOLARWIND, true, M>(n_lanes, d_launch, st, mid) : launch_gc_bg<R, SPX_BG_SOLARWIND, false, M>(n_lanes, d_launch, st, mid);
+      return xd ? launch_gc_bg<R, SPX_BG_SOLARWIND, true, M>(S, d_launch, st, mid) : launch_gc_bg<R, SPX_BG_SOLARWIND, false, M>(S, d_launch, st, mid);
    case SPX_BG_UNIFORM:
-      return xd ? launch_gc_bg<R, SPX_BG_UNIFORM, true, M>(n_lanes, d_launch, st, mid) : launch_gc_bg<R, SPX_BG_UNIFORM, false, M>(n_lanes, d_launch, st, mid);
-   case SPX_BG_GRID: return xd ? hipErrorInvalidValue : launch_gc_bg<R, SPX_BG_GRID, false, M>(n_lanes, d_launch, st, mid);
-   case SPX_BG_SHOCK: return xd ? hipErrorInvalidValue : launch_gc_bg<R, SPX_BG_SHOCK, false, M>(n_lanes, d_launch, st, mid);
-   case SPX_BG_SMOOTHSHOCK: return xd ? hipErrorInvalidValue : launch_gc_bg<R, SPX_BG_SMOOTHSHOCK, false, M>(n_lanes, d_launch, st, mid);
+      return xd ? launch_gc_bg<R, SPX_BG_UNIFORM, true, M>(S, d_launch, st, mid) : launch_gc_bg<R, SPX_BG_UNIFORM, false, M>(S, d_launch, st, mid);
+   case SPX_BG_GRID: return xd ? hipErrorInvalidValue : launch_gc_bg<R, SPX_BG_GRID, false, M>(S, d_launch, st, mid);
+   case SPX_BG_SHOCK: return xd ? hipErrorInvalidValue : launch_gc_bg<R, SPX_BG_SHOCK, false, M>(S, d_launch, st, mid);
+   case SPX_BG_SMOOTHSHOCK: return xd ? hipErrorInvalidValue : launch_gc_bg<R, SPX_BG_SMOOTHSHOCK, false, M>(S, d_launch, st, mid);
    default: return hipErrorInvalidValue;
    }
 }

@@ -70,6 +70,23 @@ struct Launch {
    int32_t* ev_bnd;                     // 3 * n_lanes
    int32_t* ev_pending;                 // bit per class
    int32_t* ex_code;                    // discard reason of the last step kernel
+   // compaction (LaunchShape::list): the place of each running slot among its query's, the running slots of each
+   // query counted by the service kernel (two sets of n_queries, used in turn), and the list of running slots
+   int32_t* rank;
+   uint32_t* n_running;
+   int32_t* list;
+   int32_t n_queries, pad_;             // size of the query table
+};
+
+// What one engine launch covers.
+struct LaunchShape {
+   uint64_t span = 0;                   // slots the service kernel covers: the first `span`, whole blocks
+   int32_t n_steps = 0;                 // steps per running slot
+   bool few = false;                    // the few-wave step kernel
+   // The step kernel takes the running slots from a list that packs them into full waves, a query's in consecutive
+   // places from a wave boundary; -1: the slots in place.  0 or 1 picks the set of n_running the launch uses.
+   int32_t packed = -1;
+   uint64_t list_span = 0;              // list places the step kernel covers (whole waves): at least those in use
 };
 
 // Compensated FP64 accumulation of the FP32-step kernels: the sums t, x, y, z and p (Parker) or
@@ -85,12 +102,13 @@ struct Launch {
 // A wave then issues one instruction every 4 cycles whatever its independence, so the way to a shorter step is
 // fewer instructions per lane: four lanes share a trajectory (quad_get in spx_engine.h).
 enum { LAUNCH_BOTH = 0, LAUNCH_FEW = 1, LAUNCH_SERVICE = 2 };   // dispatch templates: service + step, the few-wave step, service alone
-hipError_t launch_f64(const spx_plan_desc& host_plan, uint64_t n_lanes, const Launch* dev_launch, bool few,
-                      hipStream_t stream, hipEvent_t mid);
-hipError_t launch_f32(const spx_plan_desc& host_plan, uint64_t n_lanes, const Launch* dev_launch, bool few,
-                      hipStream_t stream, hipEvent_t mid);
-hipError_t launch_few_f64(const spx_plan_desc& host_plan, uint64_t n_lanes, const Launch* dev_launch, hipStream_t stream);
-hipError_t launch_few_f32(const spx_plan_desc& host_plan, uint64_t n_lanes, const Launch* dev_launch, hipStream_t stream);
+hipError_t launch_f64(const spx_plan_desc& host_plan, const LaunchShape& shape, const Launch* dev_launch, hipStream_t stream, hipEvent_t mid);
+hipError_t launch_f32(const spx_plan_desc& host_plan, const LaunchShape& shape, const Launch* dev_launch, hipStream_t stream, hipEvent_t mid);
+hipError_t launch_few_f64(const spx_plan_desc& host_plan, const LaunchShape& shape, const Launch* dev_launch, hipStream_t stream);
+hipError_t launch_few_f32(const spx_plan_desc& host_plan, const LaunchShape& shape, const Launch* dev_launch, hipStream_t stream);
+// The list of the running slots after a service kernel that counted them (spx_kernels_f64.hip).
+hipError_t pack_running(const LaunchShape& shape, const Launch* dev_launch, hipStream_t stream);
+
 // Which step kernels have the few-wave form.  Measured on one wave per SIMD, one pass: FP64 modulation 15.6 -> 9.4 ms
 // (64 trajectories), guiding centre 265 -> 189 ms (5000), gridded wind with anisotropic kappa 565 -> 306 ms (10^4);
 // FP32 with kappa ~ T r^2 41 -> 26 ms (2000), gridded anisotropic 289 -> 134 ms (500).
@@ -106,11 +124,11 @@ inline bool has_few(const spx_plan_desc& p, int precision)
 // corner it is, in corner order i + 2j + 4k (corners beyond the last zone repeat it; no stencil reads them).
 hipError_t grid_expand_cells(const double* zones, const int32_t nz[3], float* c32, hipStream_t st);
 
-inline hipError_t launch_transport(const spx_plan_desc& host_plan, uint64_t n_lanes, const Launch* dev_launch,
-                                   int precision, bool few, hipStream_t stream, hipEvent_t mid)
+inline hipError_t launch_transport(const spx_plan_desc& host_plan, const LaunchShape& shape, const Launch* dev_launch,
+                                   int precision, hipStream_t stream, hipEvent_t mid)
 {
-   return precision == SPX_PREC_MIXED ? launch_f32(host_plan, n_lanes, dev_launch, few, stream, mid)
-                                      : launch_f64(host_plan, n_lanes, dev_launch, few, stream, mid);
+   return precision == SPX_PREC_MIXED ? launch_f32(host_plan, shape, dev_launch, stream, mid)
+                                      : launch_f64(host_plan, shape, dev_launch, stream, mid);
 }
 
 }  // namespace spx

@@ -17,18 +17,18 @@
 
 namespace spx {
 
-hipError_t launch_f32(const spx_plan_desc& hp, uint64_t n_lanes, const Launch* d_launch, bool few, hipStream_t st, hipEvent_t mid)
+hipError_t launch_f32(const spx_plan_desc& hp, const LaunchShape& S, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
 {
    const bool parker = hp.traj_type == SPX_TRAJ_PARKER || hp.traj_type == SPX_TRAJ_PARKER_SOURCE || hp.traj_type == SPX_TRAJ_FIELDLINE;
    const bool gc = hp.traj_type >= SPX_TRAJ_GUIDING_DIFF_SCATT && hp.traj_type <= SPX_TRAJ_GUIDING_DIFF;
-   if (few && has_few(hp, SPX_PREC_MIXED)) {
-      const hipError_t e = dispatch_parker<float, LAUNCH_SERVICE>(hp, n_lanes, d_launch, st, mid);
-      return e != hipSuccess ? e : launch_few_f32(hp, n_lanes, d_launch, st);
+   if (S.few && has_few(hp, SPX_PREC_MIXED)) {
+      const hipError_t e = dispatch_parker<float, LAUNCH_SERVICE>(hp, S, d_launch, st, mid);
+      return e != hipSuccess ? e : launch_few_f32(hp, S, d_launch, st);
    }
-   if (parker) return dispatch_parker<float, LAUNCH_BOTH>(hp, n_lanes, d_launch, st, mid);
-   if (gc) return dispatch_gc<float, LAUNCH_BOTH>(hp, n_lanes, d_launch, st, mid);
-   if (hp.traj_type == SPX_TRAJ_LORENTZ) return dispatch_lorentz<float>(hp, n_lanes, d_launch, st, mid);
-   if (hp.traj_type == SPX_TRAJ_FOCUSED) return dispatch_focused<float>(hp, n_lanes, d_launch, st, mid);
+   if (parker) return dispatch_parker<float, LAUNCH_BOTH>(hp, S, d_launch, st, mid);
+   if (gc) return dispatch_gc<float, LAUNCH_BOTH>(hp, S, d_launch, st, mid);
+   if (hp.traj_type == SPX_TRAJ_LORENTZ) return dispatch_lorentz<float>(hp, S, d_launch, st, mid);
+   if (hp.traj_type == SPX_TRAJ_FOCUSED) return dispatch_focused<float>(hp, S, d_launch, st, mid);
    return hipErrorInvalidValue;
 }
 

@@ -118,10 +118,10 @@ __device__ int lz_set_start(PlanPtr P, QueryPtr Q, LaunchPtr L, const spx_rng_de
 }
 
 template <typename R, int BG>
-__global__ __launch_bounds__(BLOCK) void lz_service(const Launch* __restrict__ Lg)
+__global__ __launch_bounds__(BLOCK) void lz_service(const Launch* __restrict__ Lg, int32_t packed)
 {
    const LaunchPtr L = (LaunchPtr)Lg;
-   service_slot(L, [&](PlanPtr P, QueryPtr Q, const spx_rng_desc& rng, uint64_t slot, uint64_t traj, uint32_t& nu) {
+   service_slot(L, packed, [&](PlanPtr P, QueryPtr Q, const spx_rng_desc& rng, uint64_t slot, uint64_t traj, uint32_t& nu) {
       return lz_set_start<R, BG>(P, Q, L, rng, slot, traj, nu);
    });
 }
@@ -185,14 +185,17 @@ __device__ __forceinline__ int lz_step(PlanPtr P, LaunchPtr L, uint64_t slot, Lz
 }
 
 template <typename R, int BG, int FWD>
-__global__ __launch_bounds__(BLOCK) void lz_step_kernel(const Launch* __restrict__ Lg)
+__global__ __launch_bounds__(BLOCK) void lz_step_kernel(const Launch* __restrict__ Lg, int32_t packed, int32_t n_steps)
 {
    const LaunchPtr Lp = (LaunchPtr)Lg;
    __shared__ ColdLDS C;
    const int tid = threadIdx.x;
-   const uint64_t slot = (uint64_t)blockIdx.x * BLOCK + tid;
+   const int32_t place = slot_of<0>(Lp, packed);
+   const int32_t place0 = __builtin_amdgcn_readfirstlane(place);
+   if (place0 < 0) return;
+   const uint64_t slot = place < 0 ? (uint64_t)place0 : (uint64_t)place;
    const int q = __builtin_amdgcn_readfirstlane(Lp->slot_q[slot]);
-   const bool run = q >= 0 && Lp->active[slot] == SLOT_RUN;
+   const bool run = q >= 0 && place >= 0 && Lp->active[slot] == SLOT_RUN;
    if (__ballot(run) == 0) return;
    const QueryPtr Q = query_of(Lp, q);
    const PlanPtr P = plan_of(Q);
@@ -215,7 +218,7 @@ __global__ __launch_bounds__(BLOCK) void lz_step_kernel(const Launch* __restrict
    int st = run ? SLOT_RUN : SLOT_IDLE;
    int exc = 0;
    unsigned long long steps_here = 0;
-   for (int it = 0; it < Lp->steps_per_launch; it++) {
+   for (int it = 0; it < n_steps; it++) {
       if (__ballot(st == SLOT_RUN) == 0) break;
       if (st != SLOT_RUN) continue;
       PlanPtr Pi = P;
@@ -251,31 +254,34 @@ __global__ __launch_bounds__(BLOCK) void lz_step_kernel(const Launch* __restrict
 }
 
 template <typename R, int BG, int FWD>
-static hipError_t launch_lz_bg(uint64_t n_lanes, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
+static hipError_t launch_lz_bg(const LaunchShape& S, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
 {
-   const unsigned grid = (unsigned)((n_lanes + BLOCK - 1) / BLOCK);
-   hipLaunchKernelGGL((lz_service<R, BG>), dim3(grid), dim3(BLOCK), 0, st, d_launch);
+   hipLaunchKernelGGL((lz_service<R, BG>), dim3(service_grid(S)), dim3(BLOCK), 0, st, d_launch, S.packed);
+   if (S.packed >= 0) {
+      hipError_t e = pack_running(S, d_launch, st);
+      if (e != hipSuccess) return e;
+   }
    if (mid) {
       hipError_t e = hipEventRecord(mid, st);
       if (e != hipSuccess) return e;
    }
-   hipLaunchKernelGGL((lz_step_kernel<R, BG, FWD>), dim3(grid), dim3(BLOCK), 0, st, d_launch);
+   hipLaunchKernelGGL((lz_step_kernel<R, BG, FWD>), dim3(step_grid<0>(S)), dim3(BLOCK), 0, st, d_launch, S.packed, S.n_steps);
    return hipGetLastError();
 }
 
 template <typename R>
-hipError_t dispatch_lorentz(const spx_plan_desc& hp, uint64_t n_lanes, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
+hipError_t dispatch_lorentz(const spx_plan_desc& hp, const LaunchShape& S, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
 {
    const bool fwd = hp.time_flow == 0;
    switch (hp.bg.kind) {
    case SPX_BG_SOLARWIND:
-      return fwd ? launch_lz_bg<R, SPX_BG_SOLARWIND, 1>(n_lanes, d_launch, st, mid) : launch_lz_bg<R, SPX_BG_SOLARWIND, 0>(n_lanes, d_launch, st, mid);
+      return fwd ? launch_lz_bg<R, SPX_BG_SOLARWIND, 1>(S, d_launch, st, mid) : launch_lz_bg<R, SPX_BG_SOLARWIND, 0>(S, d_launch, st, mid);
    case SPX_BG_UNIFORM:
-      return fwd ? launch_lz_bg<R, SPX_BG_UNIFORM, 1>(n_lanes, d_launch, st, mid) : launch_lz_bg<R, SPX_BG_UNIFORM, 0>(n_lanes, d_launch, st, mid);
+      return fwd ? launch_lz_bg<R, SPX_BG_UNIFORM, 1>(S, d_launch, st, mid) : launch_lz_bg<R, SPX_BG_UNIFORM, 0>(S, d_launch, st, mid);
    case SPX_BG_SHOCK:
-      return fwd ? launch_lz_bg<R, SPX_BG_SHOCK, 1>(n_lanes, d_launch, st, mid) : launch_lz_bg<R, SPX_BG_SHOCK, 0>(n_lanes, d_launch, st, mid);
+      return fwd ? launch_lz_bg<R, SPX_BG_SHOCK, 1>(S, d_launch, st, mid) : launch_lz_bg<R, SPX_BG_SHOCK, 0>(S, d_launch, st, mid);
    case SPX_BG_GRID:
-      return fwd ? launch_lz_bg<R, SPX_BG_GRID, 1>(n_lanes, d_launch, st, mid) : launch_lz_bg<R, SPX_BG_GRID, 0>(n_lanes, d_launch, st, mid);
+      return fwd ? launch_lz_bg<R, SPX_BG_GRID, 1>(S, d_launch, st, mid) : launch_lz_bg<R, SPX_BG_GRID, 0>(S, d_launch, st, mid);
    default: return hipErrorInvalidValue;
    }
 }

@@ -265,10 +265,10 @@ __device__ int parker_set_start(PlanPtr P, QueryPtr Q, LaunchPtr L, const spx_rn
 }
 
 template <typename R, int BG, int TT>
-__global__ __launch_bounds__(BLOCK) void parker_service(const Launch* __restrict__ Lg)
+__global__ __launch_bounds__(BLOCK) void parker_service(const Launch* __restrict__ Lg, int32_t packed)
 {
    const LaunchPtr L = (LaunchPtr)Lg;
-   service_slot(L, [&](PlanPtr P, QueryPtr Q, const spx_rng_desc& rng, uint64_t slot, uint64_t traj, uint32_t& nu) {
+   service_slot(L, packed, [&](PlanPtr P, QueryPtr Q, const spx_rng_desc& rng, uint64_t slot, uint64_t traj, uint32_t& nu) {
       return parker_set_start<R, BG, TT>(P, Q, L, rng, slot, traj, nu);
    });
 }
@@ -603,17 +603,20 @@ __device__ __forceinline__ int parker_step(PP P, PlanPtr Pc, LaunchPtr L, const 
 }
 
 template <typename R, int BG, int FWD, int TT, int DF, int V>
-__device__ __forceinline__ void parker_step_body(const Launch* __restrict__ Lg)
+__device__ __forceinline__ void parker_step_body(const Launch* __restrict__ Lg, int32_t packed, int32_t n_steps)
 {
    const LaunchPtr Lp = (LaunchPtr)Lg;
    __shared__ ColdLDS C;
    const int tid = threadIdx.x;
    __shared__ RingLDS<R, V> ring;
-   const uint64_t slot = slot_of<V>();
+   const int32_t place = slot_of<V>(Lp, packed);
+   const int32_t place0 = __builtin_amdgcn_readfirstlane(place);
+   if (place0 < 0) return;
+   const uint64_t slot = place < 0 ? (uint64_t)place0 : (uint64_t)place;
    const bool writer = slot_writer<V>();
    // the slots of a wave work for one query (the pool size is a multiple of the block size)
    const int q = __builtin_amdgcn_readfirstlane(Lp->slot_q[slot]);
-   const bool run = q >= 0 && Lp->active[slot] == SLOT_RUN;
+   const bool run = q >= 0 && place >= 0 && Lp->active[slot] == SLOT_RUN;
    if (__ballot(run) == 0) return;
    const QueryPtr Q = query_of(Lp, q);
    const PlanPtr P = plan_of(Q);
@@ -652,7 +655,6 @@ __device__ __forceinline__ void parker_step_body(const Launch* __restrict__ Lg)
    unsigned long long steps_here = 0;
    HotPlan<R> hot;
    if constexpr (V == 1 && !is_f32<R>()) load_hot(hot, P);
-   const int n_steps = Lp->steps_per_launch;
    for (int it = 0; it < n_steps; it++) {
       if (__ballot(st == SLOT_RUN) == 0) break;
       if (st != SLOT_RUN) continue;
@@ -723,9 +725,9 @@ constexpr int pk_waves()
 }
 template <typename R, int BG, int FWD, int TT, int DF, int V>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(V == 1 ? 1 : pk_waves<R, BG, TT, DF>())))
-void parker_step_kernel(const Launch* __restrict__ Lg)
+void parker_step_kernel(const Launch* __restrict__ Lg, int32_t packed, int32_t n_steps)
 {
-   parker_step_body<R, BG, FWD, TT, DF, V>(Lg);
+   parker_step_body<R, BG, FWD, TT, DF, V>(Lg, packed, n_steps);
 }
 
 // The gridded background's step kernel waits on gathers: its V = 0 form asks the compiler for room for
@@ -734,20 +736,23 @@ void parker_step_kernel(const Launch* __restrict__ Lg)
 #define SPX_GRID_WAVES 1
 #endif
 template <typename R, int FWD, int TT, int V>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(V == 1 ? 1 : SPX_GRID_WAVES))) void parker_grid_step_kernel(const Launch* __restrict__ Lg)
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(V == 1 ? 1 : SPX_GRID_WAVES))) void parker_grid_step_kernel(const Launch* __restrict__ Lg, int32_t packed, int32_t n_steps)
 {
-   parker_step_body<R, SPX_BG_GRID, FWD, TT, 0, V>(Lg);
+   parker_step_body<R, SPX_BG_GRID, FWD, TT, 0, V>(Lg, packed, n_steps);
 }
 
 // ---------------------------------------------------------------------------------------------
 // Dispatch: one engine launch = service kernel + step kernel on the same stream (M: spx_kernels.h)
 // ---------------------------------------------------------------------------------------------
 template <typename R, int BG, int FWD, int TT, int DF, int M>
-static hipError_t launch_parker(uint64_t n_lanes, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
+static hipError_t launch_parker(const LaunchShape& S, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
 {
-   const unsigned grid = (unsigned)((n_lanes + BLOCK - 1) / BLOCK);   // n_lanes: the slots that may hold a trajectory
    if constexpr (M != LAUNCH_FEW) {
-      hipLaunchKernelGGL((parker_service<R, BG, TT>), dim3(grid), dim3(BLOCK), 0, st, d_launch);
+      hipLaunchKernelGGL((parker_service<R, BG, TT>), dim3(service_grid(S)), dim3(BLOCK), 0, st, d_launch, S.packed);
+      if (S.packed >= 0) {
+         hipError_t e = pack_running(S, d_launch, st);
+         if (e != hipSuccess) return e;
+      }
       if (mid) {
          hipError_t e = hipEventRecord(mid, st);
          if (e != hipSuccess) return e;
@@ -755,54 +760,54 @@ static hipError_t launch_parker(uint64_t n_lanes, const Launch* d_launch, hipStr
    }
    if constexpr (M != LAUNCH_SERVICE) {
       constexpr int V = (M == LAUNCH_FEW) ? 1 : 0;
-      const unsigned sg = V == 1 ? grid * QUAD : grid;
-      if constexpr (BG == SPX_BG_GRID) hipLaunchKernelGGL((parker_grid_step_kernel<R, FWD, TT, V>), dim3(sg), dim3(BLOCK), 0, st, d_launch);
-      else hipLaunchKernelGGL((parker_step_kernel<R, BG, FWD, TT, DF, V>), dim3(sg), dim3(BLOCK), 0, st, d_launch);
+      const unsigned sg = step_grid<V>(S);
+      if constexpr (BG == SPX_BG_GRID) hipLaunchKernelGGL((parker_grid_step_kernel<R, FWD, TT, V>), dim3(sg), dim3(BLOCK), 0, st, d_launch, S.packed, S.n_steps);
+      else hipLaunchKernelGGL((parker_step_kernel<R, BG, FWD, TT, DF, V>), dim3(sg), dim3(BLOCK), 0, st, d_launch, S.packed, S.n_steps);
    }
    return hipGetLastError();
 }
 
 template <typename R, int BG, int FWD, int TT, int M>
-static hipError_t dispatch_df(const spx_plan_desc& hp, uint64_t n_lanes, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
+static hipError_t dispatch_df(const spx_plan_desc& hp, const LaunchShape& S, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
 {
    switch (hp.df.kind) {
-   case SPX_DF_RIGBMAG: return launch_parker<R, BG, FWD, TT, SPX_DF_RIGBMAG, M>(n_lanes, d_launch, st, mid);
-   case SPX_DF_FULL: return launch_parker<R, BG, FWD, TT, SPX_DF_FULL, M>(n_lanes, d_launch, st, mid);
-   default: return launch_parker<R, BG, FWD, TT, 0, M>(n_lanes, d_launch, st, mid);
+   case SPX_DF_RIGBMAG: return launch_parker<R, BG, FWD, TT, SPX_DF_RIGBMAG, M>(S, d_launch, st, mid);
+   case SPX_DF_FULL: return launch_parker<R, BG, FWD, TT, SPX_DF_FULL, M>(S, d_launch, st, mid);
+   default: return launch_parker<R, BG, FWD, TT, 0, M>(S, d_launch, st, mid);
    }
 }
 
 template <typename R, int BG, int M>
-static hipError_t dispatch_flow(const spx_plan_desc& hp, uint64_t n_lanes, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
+static hipError_t dispatch_flow(const spx_plan_desc& hp, const LaunchShape& S, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
 {
    const bool fwd = hp.time_flow == 0;
-   if (hp.traj_type == 1) return fwd ? dispatch_df<R, BG, 1, 1, M>(hp, n_lanes, d_launch, st, mid) : dispatch_df<R, BG, 0, 1, M>(hp, n_lanes, d_launch, st, mid);
+   if (hp.traj_type == 1) return fwd ? dispatch_df<R, BG, 1, 1, M>(hp, S, d_launch, st, mid) : dispatch_df<R, BG, 0, 1, M>(hp, S, d_launch, st, mid);
    if (hp.traj_type == SPX_TRAJ_FIELDLINE)
-      return fwd ? launch_parker<R, BG, 1, 2, 0, M>(n_lanes, d_launch, st, mid) : launch_parker<R, BG, 0, 2, 0, M>(n_lanes, d_launch, st, mid);
-   return fwd ? dispatch_df<R, BG, 1, 0, M>(hp, n_lanes, d_launch, st, mid) : dispatch_df<R, BG, 0, 0, M>(hp, n_lanes, d_launch, st, mid);
+      return fwd ? launch_parker<R, BG, 1, 2, 0, M>(S, d_launch, st, mid) : launch_parker<R, BG, 0, 2, 0, M>(S, d_launch, st, mid);
+   return fwd ? dispatch_df<R, BG, 1, 0, M>(hp, S, d_launch, st, mid) : dispatch_df<R, BG, 0, 0, M>(hp, S, d_launch, st, mid);
 }
 
 // The gridded background runs the generic diffusion dispatch only (every class through kappa01).
 template <typename R, int M>
-static hipError_t dispatch_grid(const spx_plan_desc& hp, uint64_t n_lanes, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
+static hipError_t dispatch_grid(const spx_plan_desc& hp, const LaunchShape& S, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
 {
    const bool fwd = hp.time_flow == 0;
    constexpr int G = SPX_BG_GRID;
-   if (hp.traj_type == 1) return fwd ? launch_parker<R, G, 1, 1, 0, M>(n_lanes, d_launch, st, mid) : launch_parker<R, G, 0, 1, 0, M>(n_lanes, d_launch, st, mid);
+   if (hp.traj_type == 1) return fwd ? launch_parker<R, G, 1, 1, 0, M>(S, d_launch, st, mid) : launch_parker<R, G, 0, 1, 0, M>(S, d_launch, st, mid);
    if (hp.traj_type == SPX_TRAJ_FIELDLINE)
-      return fwd ? launch_parker<R, G, 1, 2, 0, M>(n_lanes, d_launch, st, mid) : launch_parker<R, G, 0, 2, 0, M>(n_lanes, d_launch, st, mid);
-   return fwd ? launch_parker<R, G, 1, 0, 0, M>(n_lanes, d_launch, st, mid) : launch_parker<R, G, 0, 0, 0, M>(n_lanes, d_launch, st, mid);
+      return fwd ? launch_parker<R, G, 1, 2, 0, M>(S, d_launch, st, mid) : launch_parker<R, G, 0, 2, 0, M>(S, d_launch, st, mid);
+   return fwd ? launch_parker<R, G, 1, 0, 0, M>(S, d_launch, st, mid) : launch_parker<R, G, 0, 0, 0, M>(S, d_launch, st, mid);
 }
 
 template <typename R, int M>
-hipError_t dispatch_parker(const spx_plan_desc& hp, uint64_t n_lanes, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
+hipError_t dispatch_parker(const spx_plan_desc& hp, const LaunchShape& S, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
 {
    switch (hp.bg.kind) {
-   case SPX_BG_GRID: return dispatch_grid<R, M>(hp, n_lanes, d_launch, st, mid);
-   case SPX_BG_SOLARWIND: return dispatch_flow<R, SPX_BG_SOLARWIND, M>(hp, n_lanes, d_launch, st, mid);
-   case SPX_BG_SMOOTHSHOCK: return dispatch_flow<R, SPX_BG_SMOOTHSHOCK, M>(hp, n_lanes, d_launch, st, mid);
-   case SPX_BG_SHOCK: return dispatch_flow<R, SPX_BG_SHOCK, M>(hp, n_lanes, d_launch, st, mid);
-   case SPX_BG_UNIFORM: return dispatch_flow<R, SPX_BG_UNIFORM, M>(hp, n_lanes, d_launch, st, mid);
+   case SPX_BG_GRID: return dispatch_grid<R, M>(hp, S, d_launch, st, mid);
+   case SPX_BG_SOLARWIND: return dispatch_flow<R, SPX_BG_SOLARWIND, M>(hp, S, d_launch, st, mid);
+   case SPX_BG_SMOOTHSHOCK: return dispatch_flow<R, SPX_BG_SMOOTHSHOCK, M>(hp, S, d_launch, st, mid);
+   case SPX_BG_SHOCK: return dispatch_flow<R, SPX_BG_SHOCK, M>(hp, S, d_launch, st, mid);
+   case SPX_BG_UNIFORM: return dispatch_flow<R, SPX_BG_UNIFORM, M>(hp, S, d_launch, st, mid);
    default: return hipErrorInvalidValue;
    }
 }

@@ -168,6 +168,7 @@ hipError_t Pool::init(const spx_plan_desc& s, int prec, uint64_t lanes, int spl,
    for (auto* b : dv) TRY(b->alloc(n));
    TRY(bdelta.alloc(n * SPX_MAX_BND)); TRY(bdelta_old.alloc(n * SPX_MAX_BND));
    TRY(traj.alloc(n)); TRY(nn.alloc(n)); TRY(nu.alloc(n)); TRY(steps.alloc(n)); TRY(kc.alloc(n * SPX_KC));
+   TRY(rank.alloc(n)); TRY(list.alloc(n + 64 * (uint64_t)cap)); TRY(n_running.alloc(2 * (size_t)cap));
    TRY(queries.alloc((size_t)cap));
    TRY(queue.alloc((size_t)cap));
    TRY(d_launch.alloc(1));
@@ -189,6 +190,7 @@ hipError_t Pool::init(const spx_plan_desc& s, int prec, uint64_t lanes, int spl,
    host.t0 = t0.p; host.x0 = x0.p; host.y0 = y0.p; host.z0 = z0.p; host.m00 = m00.p; host.m01 = m01.p; host.m02 = m02.p;
    host.ev_bin = ev_bin.p; host.ev_w = ev_w.p;
    host.evs = evs.p; host.ev_bnd = ev_bnd.p; host.ev_pending = ev_pending.p; host.ex_code = ex_code.p;
+   host.rank = rank.p; host.n_running = n_running.p; host.list = list.p; host.n_queries = cap;
    TRY(reset_slots());
    return hipSuccess;
 }
@@ -198,6 +200,10 @@ hipError_t Pool::reset_slots()
    TRY(hipMemsetAsync(active.p, 0, sizeof(int32_t) * n_lanes, stream));          // SLOT_IDLE
    TRY(hipMemsetAsync(slot_q.p, 0xff, sizeof(int32_t) * n_lanes, stream));       // -1: no query
    TRY(hipMemsetAsync(ev_pending.p, 0, sizeof(int32_t) * n_lanes, stream));
+   TRY(hipMemsetAsync(n_running.p, 0, sizeof(uint32_t) * 2 * (size_t)qcap, stream));
+   turn = 0;
+   ms_per_step = round_ms = 0.0;
+   round_live = 0;
    host_queue.clear();
    std::fill(qused.begin(), qused.end(), 0);
    return upload_launch();
@@ -246,13 +252,34 @@ hipError_t Pool::remove_queue(int q)
    return upload_launch();
 }
 
-hipError_t Pool::enqueue(int n, uint64_t live)
+LaunchShape Pool::shape(uint64_t live, bool claimed, int n_steps)
+{
+   LaunchShape S;
+   S.span = span;
+   S.n_steps = n_steps;
+   // Packing pays once slots run dry and the waves outnumber the SIMDs: with at most a wave per SIMD a launch lasts
+   // as long as its longest wave however few lanes run in it.  Whole runs, one pass with the drain in place and packed:
+   // FP64 modulation 10^5 301 -> 120 ms, mixed 3*10^5 432 -> 277 ms, kappa ~ T r^2 FP64 30000 112 -> 69 ms and mixed
+   // 5*10^5 127 -> 86 ms, FP64 shock 20000 1355 -> 716 ms (the waves fit the four-lane form once packed).
+   const uint64_t full = few_limit() * 4;
+   if (claimed && span > full / 4 && live < span - span / 8) S.packed = 0;
+   const uint64_t used = S.packed >= 0 ? std::min(live, span) : span;
+   S.few = has_few(sig, precision) && used <= few_limit();
+   if (S.packed >= 0 && !S.few && span <= full) S.packed = -1;
+   if (S.packed >= 0) S.list_span = (used + 63) / 64 * 64 + (uint64_t)64 * host_queue.size();
+   return S;
+}
+
+hipError_t Pool::enqueue(int n, const LaunchShape& S0)
 {
    if (graph_launches > 0) {
       if (!graph_exec) {
+         LaunchShape G;
+         G.span = n_lanes;
+         G.n_steps = steps_per_launch;
          TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
          for (int i = 0; i < graph_launches; i++) {
-            hipError_t e = launch_transport(sig, n_lanes, d_launch.p, precision, false, stream, nullptr);
+            hipError_t e = launch_transport(sig, G, d_launch.p, precision, stream, nullptr);
             if (e != hipSuccess) {
                hipGraph_t g;
                (void)hipStreamEndCapture(stream, &g);
@@ -267,16 +294,28 @@ hipError_t Pool::enqueue(int n, uint64_t live)
       launches += (int64_t)reps * graph_launches;
       return hipSuccess;
    }
-   for (int i = 0; i < n; i++) TRY(launch_transport(sig, span, d_launch.p, precision, few(live), stream, nullptr));
+   LaunchShape S = S0;
+   for (int i = 0; i < n; i++) {
+      take_turn(S);
+      TRY(launch_transport(sig, S, d_launch.p, precision, stream, nullptr));
+   }
    launches += n;
    return hipSuccess;
 }
 
-hipError_t Pool::launch(int n, uint64_t live, float* ms_out)
+void Pool::take_turn(LaunchShape& S)
 {
+   if (S.packed < 0) return;
+   S.packed = turn;
+   turn = 1 - turn;
+}
+
+hipError_t Pool::launch(int n, const LaunchShape& S0, float* ms_out)
+{
+   LaunchShape S = S0;
    TRY(hipEventRecord(ev0, stream));
    if (graph_launches > 0) {
-      TRY(enqueue(n, live));
+      TRY(enqueue(n, S));
    }
    else {
       while (tev.size() < (size_t)2 * n) {
@@ -286,7 +325,8 @@ hipError_t Pool::launch(int n, uint64_t live, float* ms_out)
       }
       for (int i = 0; i < n; i++) {
          TRY(hipEventRecord(tev[2 * i], stream));
-         TRY(launch_transport(sig, span, d_launch.p, precision, few(live), stream, tev[2 * i + 1]));
+         take_turn(S);
+         TRY(launch_transport(sig, S, d_launch.p, precision, stream, tev[2 * i + 1]));
       }
       launches += n;
    }
@@ -307,14 +347,38 @@ hipError_t Pool::launch(int n, uint64_t live, float* ms_out)
    return hipSuccess;
 }
 
+hipError_t Pool::round(uint64_t live, bool claimed, double& ms_total, int& n_launches)
+{
+   // Looking at the counters costs some 30 us; 4 ms between looks keep that below 1% and let a drain pack its slots
+   // soon after they empty.  While trajectories barely end there is nothing to react to: the rounds grow.
+   constexpr double base_ms = 4.0, most_ms = 32.0;
+   if (live != round_live && (double)live < 0.97 * (double)round_live) round_ms = base_ms;
+   else round_ms = std::min(most_ms, round_ms > 0.0 ? 2.0 * round_ms : base_ms);
+   round_live = live;
+   int n = 1, steps = steps_per_launch;
+   if (graph_launches == 0 && ms_per_step > 0.0) {
+      const double want = round_ms / ms_per_step;   // steps
+      // short launches only where the empty slots cannot be refilled
+      if (claimed && want < steps) steps = std::max(std::min(steps, 100), (int)want);
+      n = std::max(1, std::min(8, (int)(want / steps)));
+   }
+   float ms = 0.f;
+   TRY(launch(n, shape(live, claimed, steps), &ms));
+   ms_per_step = graph_launches == 0 ? (double)ms / ((double)n * steps) : 0.0;
+   ms_total += ms;
+   n_launches += n;
+   return hipSuccess;
+}
+
 void Pool::release()
 {
    if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
    if (graph) (void)hipGraphDestroy(graph);
    graph_exec = nullptr;
    graph = nullptr;
-   DevBuf<int32_t>* di[] = {&active, &slot_q, &bcross, &bstat, &attempt, &n_events, &ev_bin, &ev_bnd, &ev_pending, &ex_code, &queue};
+   DevBuf<int32_t>* di[] = {&active, &slot_q, &bcross, &bstat, &attempt, &n_events, &ev_bin, &ev_bnd, &ev_pending, &ex_code, &queue, &rank, &list};
    for (auto* b : di) b->release();
+   n_running.release();
    DevBuf<double>* dv[] = {&t, &x, &y, &z, &m0, &m1, &m2, &amp, &wgt, &dt_prev, &src_old, &ds_prev, &dmax, &dt_adapt, &pf, &bdelta,
                            &bdelta_old, &t0, &x0, &y0, &z0, &m00, &m01, &m02, &ev_w, &evs};
    for (auto* b : dv) b->release();

@@ -92,6 +92,8 @@ struct Pool {
    DevBuf<int64_t> steps;
    DevBuf<QueryDesc> queries;
    DevBuf<int32_t> queue;
+   DevBuf<int32_t> rank, list;          // packed launches
+   DevBuf<uint32_t> n_running;
    DevBuf<Launch> d_launch;
    Launch host{};
    std::vector<int32_t> host_queue;     // admitted query indices, oldest first
@@ -110,17 +112,25 @@ struct Pool {
    hipError_t set_query(int q, const QueryDesc& d);
    hipError_t push_queue(int q, uint64_t n_traj);
    hipError_t remove_queue(int q);
-   // enqueue n engine launches on the pool's stream (graph replays when graph_launches > 0); `live` bounds the
-   // trajectories that are running or still to be claimed, and picks the step kernel's form.  The kernels cover
-   // the first `span` slots only: as many as the queries admitted since the pool was last empty can fill.
-   hipError_t enqueue(int n, uint64_t live);
+   // The shape of the next launches.  `live` bounds the trajectories that are running or still to be claimed;
+   // `claimed`: every one has been handed out, so slots that finish stay empty.
+   LaunchShape shape(uint64_t live, bool claimed, int n_steps);
+   // enqueue n engine launches on the pool's stream (graph replays of the whole pool when graph_launches > 0)
+   hipError_t enqueue(int n, const LaunchShape& S);
    // enqueue, wait, and account kernel time (ms of the call, step / service kernel split)
-   hipError_t launch(int n, uint64_t live, float* ms);
+   hipError_t launch(int n, const LaunchShape& S, float* ms);
+   // One round of a run that is waited for: enough launches, or a launch of few enough steps, that the host looks
+   // at the counters about every `round_ms`.  Adds to ms and launches.
+   hipError_t round(uint64_t live, bool claimed, double& ms, int& n_launches);
    void release();
 
 private:
    hipError_t upload_launch();
-   bool few(uint64_t live) const { return has_few(sig, precision) && std::max(live, span) <= few_limit(); }
+   void take_turn(LaunchShape& S);
+   int turn = 0;                        // the set of n_running the next packed launch uses
+   double ms_per_step = 0.0;            // of the last round, and what it was asked to last
+   double round_ms = 0.0;
+   uint64_t round_live = 0;
 };
 
 }  // namespace spx

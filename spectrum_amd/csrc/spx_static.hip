@@ -197,14 +197,16 @@ hipError_t static_run(const spx_plan_desc& plan, int precision, int steps_per_la
    // a trajectory needs at most max_attempts * (max_steps + 1) steps; a healthy run never reaches this
    const double guard = 64.0 + (double)plan.max_attempts * ((double)plan.max_steps + 1.0) / steps_per_launch *
                                    (1.0 + (double)n_traj / (double)n);
-   const uint64_t span = n_traj < n ? (n_traj + 255) / 256 * 256 : n;   // the slots the run can fill
+   LaunchShape shape;
+   shape.span = n_traj < n ? (n_traj + 255) / 256 * 256 : n;   // the slots the run can fill
+   shape.n_steps = steps_per_launch;
+   shape.few = has_few(plan, precision) && shape.span <= few_limit();
    int launches = 0, batch = 1;
    while (true) {
       TRY(hipMemcpy(&ctl, R.ctl, sizeof(ctl), hipMemcpyDeviceToHost));
       if (ctl.done >= n_traj) break;
       if (launches > guard) return hipErrorLaunchTimeOut;
-      const bool few = has_few(plan, precision) && span <= few_limit();
-      for (int i = 0; i < batch; i++) TRY(launch_transport(plan, span, R.launch, precision, few, nullptr, nullptr));
+      for (int i = 0; i < batch; i++) TRY(launch_transport(plan, shape, R.launch, precision, nullptr, nullptr));
       launches += batch;
       if (batch < 8) batch *= 2;
    }
