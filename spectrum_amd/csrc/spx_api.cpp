@@ -550,6 +550,9 @@ static void finalize_plan(spx_sim* s)
       f.sw_kg = g.ep_diag ? (float)(g.eprime[0][0] * g.eprime[1][1] * g.w0 / g.ur0) : 0.0f;
       // |B| = |B0| r_ref^2 |w| / r^3 with |w| >= r, so |B| >= |B0| r_ref^2 / r^2
       const double r2_ok = std::fabs(g.B0[0] * g.r_ref * g.r_ref) / sp_tiny_h;
+      P.bg.sw_r2_ok = 0.99 * r2_ok;
+      P.bg.sw_r2_min = 1.0e-6 * g.r_ref * g.r_ref;
+      f.sw_r2_min = (float)P.bg.sw_r2_min;
       f.sw_r2_ok = r2_ok > (double)FLT_MAX ? INFINITY : (float)r2_ok;
    }
    spx_df_t<double>& d = P.df;
@@ -558,8 +561,9 @@ static void finalize_plan(spx_sim* s)
    if (d.kind == SPX_DF_KINRAD) d.pos_dep = 1;
    if (d.kind == SPX_DF_RIGBMAG) d.pos_dep = (d.pow_law_B != 0.0);
    if (d.kind == SPX_DF_STRAUSS || d.kind == SPX_DF_POTGIETER || d.kind == SPX_DF_SOQLT) d.pos_dep = 1;   // through |B| and the region
+   d.iso_r = d.kind == SPX_DF_KINRAD && d.kap_rat == 1.0 && d.stream_dep_idx == 0;
    spx_df_t<float>& e = P.dff;
-   e.kind = d.kind; e.stream_dep_idx = d.stream_dep_idx; e.pos_dep = d.pos_dep; e.region_idx = d.region_idx;
+   e.kind = d.kind; e.stream_dep_idx = d.stream_dep_idx; e.pos_dep = d.pos_dep; e.iso_r = d.iso_r; e.region_idx = d.region_idx;
    e.lam_in = (float)d.lam_in; e.lam_out = (float)d.lam_out; e.kap_rat_in = (float)d.kap_rat_in; e.kap_rat_out = (float)d.kap_rat_out;
    e.A2A = (float)d.A2A; e.k_min = (float)d.k_min; e.ps_minus = (float)d.ps_minus;
    e.A2T = (float)d.A2T; e.A2L = (float)d.A2L; e.ps_plus = (float)d.ps_plus;

@@ -359,7 +359,60 @@ __device__ __forceinline__ int parker_step(PP P, PlanPtr Pc, LaunchPtr L, const 
    const double ydel = is_f32<R>() ? 0.0 : 1.0 / (double)delta;   // FP64: the stencil's nine quotients by delta share it
    v3<R> divK = mk<R>(R(0), R(0), R(0));
    const bool pos_dep = (DF == SPX_DF_FULL) ? false : (df.pos_dep != 0);
-   if (BG == SPX_BG_GRID && (pos_dep || K0 != K1)) {
+   // kappa isotropic and a function of |x| alone: (kappa_par - kappa_perp) b b is an exact zero at every point, so
+   // component j of div(kappa) is the difference of kappa along axis j and B is not needed there, once it is known that
+   // no point fails GetFields (its |B| < sp_tiny; on the grid the position check) or has a field that is not finite.
+   // Bit for bit the general stencil's result; the step of kappa ~ T r^2 was issue bound with two thirds of its
+   // instructions there (mixed 5*10^5 trajectories 86 -> 50 ms, FP64 30000 74 -> 47 ms; the 25^3-block grid, where only the
+   // dispatch of kappa's class and power at six points goes, mixed 2*10^5 66 -> 53 ms).
+   const bool iso = DF == 0 && df.iso_r != 0 &&
+                    (BG == SPX_BG_GRID ? PlanView<R>::bg(P).grid.fd_fields == 0
+                                       : BG == SPX_BG_SOLARWIND && sw_stencil_regular<R>(bg, rel(bg, H.x, H.y, H.z), delta));
+   if (iso) {
+      // the exponent 2 of the usual model without a branch per point; pow's code once
+      const bool square = df.pow_law_r == R(2);
+      auto axis = [&](int j, R& t) -> bool {
+         const double ex = (j == 0) ? 1.0 : 0.0, ey = (j == 1) ? 1.0 : 0.0, ez = (j == 2) ? 1.0 : 0.0;
+         double xf = H.x + (double)delta * ex, yf = H.y + (double)delta * ey, zf = H.z + (double)delta * ez;
+         bool ok = true;
+         if constexpr (BG == SPX_BG_GRID) ok = grid_inside<R>(bg.grid, xf, yf, zf);
+         const R rf = R(norm(mk<double>(xf, yf, zf))) / df.r0;
+         xf -= 2.0 * (double)delta * ex;
+         yf -= 2.0 * (double)delta * ey;
+         zf -= 2.0 * (double)delta * ez;
+         if constexpr (BG == SPX_BG_GRID) ok = ok && grid_inside<R>(bg.grid, xf, yf, zf);
+         const R rb = R(norm(mk<double>(xf, yf, zf))) / df.r0;
+         R Kf, Kb;
+         if (square) { Kf = km * (rf * rf); Kb = km * (rb * rb); }
+         else { Kf = km * rpow(rf, df.pow_law_r); Kb = km * rpow(rb, df.pow_law_r); }
+         own_rounding(Kf, Kb);
+         t = Kf - Kb;
+         return ok;
+      };
+      R t0 = R(0), t1 = R(0), t2 = R(0);
+      if constexpr (V == 1) {
+         R t;
+         if (quad_any(!axis(min(quad_lane(), 2), t))) return 1;
+         t0 = quad_get<0>(t); t1 = quad_get<1>(t); t2 = quad_get<2>(t);
+      }
+      else if (square) {
+         const bool ok0 = axis(0, t0), ok1 = axis(1, t1), ok2 = axis(2, t2);
+         if (!(ok0 && ok1 && ok2)) return 1;
+      }
+      else {
+#pragma unroll 1
+         for (int j = 0; j < 3; j++) {
+            R t;
+            if (!axis(j, t)) return 1;
+            t0 = j == 0 ? t : t0; t1 = j == 1 ? t : t1; t2 = j == 2 ? t : t2;
+         }
+      }
+      own_rounding(t0, t1, t2);
+      if constexpr (is_f32<R>()) divK = mk<R>(hdi * t0, hdi * t1, hdi * t2);
+      else divK = mk<R>(div_rn(R(0.5) * t0, delta, ydel), div_rn(R(0.5) * t1, delta, ydel), div_rn(R(0.5) * t2, delta, ydel));
+      own_rounding(divK);
+   }
+   else if (BG == SPX_BG_GRID && (pos_dep || K0 != K1)) {
       // the same stencil on the gridded background: interpolated B and |B| at the derivative points
       auto axis = [&](int j, v3<R>& t) -> bool {
          const double ex = (j == 0) ? 1.0 : 0.0, ey = (j == 1) ? 1.0 : 0.0, ez = (j == 2) ? 1.0 : 0.0;
@@ -654,7 +707,9 @@ __device__ __forceinline__ void parker_step_body(const Launch* __restrict__ Lg, 
    int exc = 0;
    unsigned long long steps_here = 0;
    HotPlan<R> hot;
-   if constexpr (V == 1 && !is_f32<R>()) load_hot(hot, P);
+   // the gridded step's plan is too large to keep (420 registers, most of them spilled: 10% slower than reading it)
+   constexpr bool HOT = V == 1 && !is_f32<R>() && BG != SPX_BG_GRID;
+   if constexpr (HOT) load_hot(hot, P);
    for (int it = 0; it < n_steps; it++) {
       if (__ballot(st == SLOT_RUN) == 0) break;
       if (st != SLOT_RUN) continue;
@@ -667,7 +722,7 @@ __device__ __forceinline__ void parker_step_body(const Launch* __restrict__ Lg, 
       asm volatile("" : "+s"(Pi));
       LaunchPtr Li = Lp;
       asm volatile("" : "+s"(Li));
-      if constexpr (V == 1 && !is_f32<R>()) {
+      if constexpr (HOT) {
          const HotPlan<R>* h = &hot;
          e = (TT == 2) ? fieldline_step<R, BG, FWD, V>(h, Pi, Li, slot, H, C, tid, bflags)
                        : parker_step<R, BG, FWD, TT, DF, V>(h, Pi, Li, rng, first, slot, H, C, tid, bflags);
@@ -731,9 +786,9 @@ void parker_step_kernel(const Launch* __restrict__ Lg, int32_t packed, int32_t n
 }
 
 // The gridded background's step kernel waits on gathers: its V = 0 form asks the compiler for room for
-// SPX_GRID_WAVES resident waves per SIMD (1: the compiler's own register budget).
+// SPX_GRID_WAVES resident waves per SIMD (FP64: 2, its 258 registers held to 256).
 #ifndef SPX_GRID_WAVES
-#define SPX_GRID_WAVES 1
+#define SPX_GRID_WAVES 2
 #endif
 template <typename R, int FWD, int TT, int V>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(V == 1 ? 1 : SPX_GRID_WAVES))) void parker_grid_step_kernel(const Launch* __restrict__ Lg, int32_t packed, int32_t n_steps)

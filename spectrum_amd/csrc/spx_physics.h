@@ -189,7 +189,7 @@ __device__ __forceinline__ void load_hot(HotPlan<R>& h, PlanPtr P)
 #define SPX_HOT(m) keep(h.vbg.m, b.m)
    SPX_HOT(kind); SPX_HOT(ep_diag); SPX_HOT(t0); SPX_HOT(r0); SPX_HOT(u0); SPX_HOT(B0); SPX_HOT(dmax0); SPX_HOT(r_ref); SPX_HOT(dmax_fraction);
    SPX_HOT(eprime[0]); SPX_HOT(eprime[1]); SPX_HOT(eprime[2]); SPX_HOT(ur0); SPX_HOT(w0); SPX_HOT(hp_rad); SPX_HOT(ur0_rcp); SPX_HOT(sw_c1);
-   SPX_HOT(sw_k); SPX_HOT(sw_kg); SPX_HOT(sw_r2_ok); SPX_HOT(n_shock); SPX_HOT(v_shock); SPX_HOT(compression); SPX_HOT(u1); SPX_HOT(B1);
+   SPX_HOT(sw_k); SPX_HOT(sw_kg); SPX_HOT(sw_r2_ok); SPX_HOT(sw_r2_min); SPX_HOT(n_shock); SPX_HOT(v_shock); SPX_HOT(compression); SPX_HOT(u1); SPX_HOT(B1);
    SPX_HOT(E0); SPX_HOT(E1); SPX_HOT(width_shock); SPX_HOT(Eu);
    SPX_HOT(grid.nb); SPX_HOT(grid.nz); SPX_HOT(grid.dom_min); SPX_HOT(grid.dom_max); SPX_HOT(grid.block_length); SPX_HOT(grid.f_len);
    SPX_HOT(grid.f_vel); SPX_HOT(grid.f_mag); SPX_HOT(grid.bmag_min); SPX_HOT(grid.inner_lo); SPX_HOT(grid.inner_hi); SPX_HOT(grid.fd_fields);
@@ -197,7 +197,7 @@ __device__ __forceinline__ void load_hot(HotPlan<R>& h, PlanPtr P)
 #undef SPX_HOT
    const spx_df_t<R>& f = hot_df(g, (R*)nullptr);
 #define SPX_HOT(m) keep(h.vdf.m, f.m)
-   SPX_HOT(kind); SPX_HOT(stream_dep_idx); SPX_HOT(pos_dep); SPX_HOT(region_idx); SPX_HOT(D0); SPX_HOT(Dperp); SPX_HOT(Dpara); SPX_HOT(kap0);
+   SPX_HOT(kind); SPX_HOT(stream_dep_idx); SPX_HOT(pos_dep); SPX_HOT(iso_r); SPX_HOT(region_idx); SPX_HOT(D0); SPX_HOT(Dperp); SPX_HOT(Dpara); SPX_HOT(kap0);
    SPX_HOT(U0); SPX_HOT(pow_law_U); SPX_HOT(p0); SPX_HOT(pow_law_p); SPX_HOT(kap_rat); SPX_HOT(T0); SPX_HOT(r0); SPX_HOT(pow_law_T);
    SPX_HOT(pow_law_r); SPX_HOT(u_up); SPX_HOT(w_sh); SPX_HOT(s_sh); SPX_HOT(dn_up_rat); SPX_HOT(lam0); SPX_HOT(R0); SPX_HOT(B0);
    SPX_HOT(pow_law_R); SPX_HOT(pow_law_B); SPX_HOT(lam_in); SPX_HOT(lam_out); SPX_HOT(kap_rat_in); SPX_HOT(kap_rat_out); SPX_HOT(A2A);
@@ -322,6 +322,15 @@ template <typename R, typename BD>
 SPX_HD bool sw_stencil_clear(BD& b, v3<R> c, R h)
 {
    return norm2(c) + h * h + (R(2) * h) * (fabs(c.x) + fabs(c.y) + fabs(c.z)) <= b.sw_r2_ok;
+}
+
+// True when, besides, no such point can meet a field that is not finite: h is at most |c| / 2, so every point keeps
+// at least |c| / 2 from the origin.
+template <typename R, typename BD>
+SPX_HD bool sw_stencil_regular(BD& b, v3<R> c, R h)
+{
+   const R c2 = norm2(c);
+   return sw_stencil_clear<R>(b, c, h) && c2 >= b.sw_r2_min && R(4) * (h * h) <= c2;
 }
 
 template <typename R, typename BD>

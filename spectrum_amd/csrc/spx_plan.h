@@ -71,7 +71,8 @@ struct spx_bg_t {
    T ur0_rcp;                          // 1 / ur0, correctly rounded (the FP64 step's quotients by ur0)
    T sw_c1, sw_k;                      // FP32 step: B0 r_ref^2 and w0 / ur0 of the closed-form spiral
    T sw_kg;                            // FP32 step: w0 / ur0 times eprime[0][0] eprime[1][1], the winding in the global frame (diagonal bases)
-   T sw_r2_ok;                         // FP32 step: |B| >= sp_tiny wherever |x - r0|^2 <= this (|B0| r_ref^2 / sp_tiny)
+   T sw_r2_ok;                         // |B| >= sp_tiny wherever |x - r0|^2 <= this (|B0| r_ref^2 / sp_tiny; FP64: 1% inside it)
+   T sw_r2_min;                        // |x - r0|^2 down to which |B| and bhat are far from overflow (r_ref 1e-3)^2
    // BackgroundShock / BackgroundSmoothShock (src/background_shock.cc:58-86, src/background_smooth_shock.cc:139-146)
    T n_shock[3], v_shock, compression, u1[3], B1[3], E0[3], E1[3], width_shock;
    // BackgroundUniform (src/background_uniform.cc:58-64)
@@ -84,6 +85,7 @@ typedef spx_bg_t<double> spx_bg_desc;
 template <typename T>
 struct spx_df_t {
    int32_t kind, stream_dep_idx, pos_dep;
+   int32_t iso_r;                       // kappa_perp == kappa_par, a function of |x| and p alone (KINRAD, kap_rat 1, no stream dependence)
    int32_t region_idx;                  // Strauss / Potgieter: LISM_idx, the region indicator read (-1: none); SOQLT: Bmix_idx
    T D0, Dperp, Dpara;
    T kap0, U0, pow_law_U, p0, pow_law_p, kap_rat;
