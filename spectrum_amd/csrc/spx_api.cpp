@@ -238,7 +238,6 @@ static int add_background(spx_sim* s, const std::string& cls, Reader& r)
       for (int k = 0; k < 3; k++)
          for (int j = 0; j < 3; j++)
             if ((j != k && g.eprime[k][j] != 0.0) || (j == k && std::fabs(g.eprime[k][j]) != 1.0)) g.ep_diag = 0;
-      if (g.ep_diag && g.eprime[0][0] == 1.0 && g.eprime[1][1] == 1.0 && g.eprime[2][2] == 1.0) g.ep_diag = 2;   // x1 is exact: skipped
       g.ur0 = std::fabs(g.u0[0]);
       g.ur0_rcp = 1.0 / g.ur0;
       g.hp_rad = 117.0 * 1.495978707E+13 / 1.0E10;

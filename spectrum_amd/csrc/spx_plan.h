@@ -63,7 +63,7 @@ template <typename T>
 struct spx_bg_t {
    typedef T real;
    int32_t kind;
-   int32_t ep_diag;                    // SolarWind: eprime is diagonal with entries +-1 (rotation axis along +-z); 2: the identity
+   int32_t ep_diag;                    // SolarWind: eprime is diagonal with entries +-1 (rotation axis along +-z)
    double t0, r0[3];                   // always double: positions are accumulated in double
    T u0[3], B0[3], dmax0;
    // BackgroundSolarWind (src/background_solarwind.cc:58-84)
