@@ -90,16 +90,6 @@ __device__ __forceinline__ bool quad_any(bool b)   // over the three axes
    const int v = b ? 1 : 0;
    return (quad_get<0>(v) | quad_get<1>(v) | quad_get<2>(v)) != 0;
 }
-template <typename R> __device__ __forceinline__ void own_rounding1(R& v) { if constexpr (is_f32<R>()) asm("" : "+v"(v)); }
-template <typename R> __device__ __forceinline__ void own_rounding1(v3<R>& v)
-{
-   own_rounding1(v.x);
-   own_rounding1(v.y);
-   own_rounding1(v.z);
-}
-// A sum whose next term follows in the same basic block: the FP32 unit contracts across statements, and without
-// this it would fuse the multiply of the term already in the sum instead of the next one's, as the loop does.
-template <typename... T> __device__ __forceinline__ void own_rounding(T&... v) { (own_rounding1(v), ...); }
 __device__ __forceinline__ int quad_lane() { return (int)threadIdx.x & (QUAD - 1); }
 // The slot of a lane in a step kernel (-1: none), and whether the lane writes for it.  The running slots come from
 // the launch's list when it is packed; a wave whose first place is empty has none.

@@ -44,7 +44,7 @@ __device__ __forceinline__ bool gc_fields(BD& bg, double t, double x, double y, 
       v3<R> U;
       R gB[6];
       double zl_min;
-      if (!grid_eval_gc<R>(bg.grid, x, y, z, U, F.B, F.Bmag, F.E, F.gradBmag, gB, zl_min)) return false;
+      if (!grid_eval_gc<R, V>(bg.grid, x, y, z, U, F.B, F.Bmag, F.E, F.gradBmag, gB, zl_min)) return false;
       F.dmax = fmin(F.dmax, R(zl_min));
       F.rg = R(0);
       if (F.Bmag < R(sp_tiny)) return false;

@@ -39,7 +39,7 @@ __device__ __forceinline__ bool parker_fields(BD& bg, double t, double x, double
    if constexpr (BG == SPX_BG_GRID) {
       // BackgroundServer: interpolated U, B and |B|, the stencil's grad U, dmax limited by the zone size
       GridFields<R> G;
-      if (!grid_eval<R, true>(bg.grid, x, y, z, G)) return false;
+      if (!grid_eval<R, true, V>(bg.grid, x, y, z, G)) return false;
       F.dmax = fmin(F.dmax, R(G.zl_min));
       F.U = G.U;
       F.Bmag = G.Bmag;
@@ -423,7 +423,7 @@ __device__ __forceinline__ int parker_step(PP P, PlanPtr Pc, LaunchPtr L, const 
          GridFields<R> Gf, Gb;
          Gf.U = Gb.U = Gf.B = Gb.B = mk<R>(R(0), R(0), R(0));
          Gf.Bmag = Gb.Bmag = H.F.Bmag;
-         if (loads ? !grid_eval<R, false>(bg.grid, xf, yf, zf, Gf) : !grid_inside<R>(bg.grid, xf, yf, zf)) return false;
+         if (loads ? !grid_eval<R, false, V>(bg.grid, xf, yf, zf, Gf) : !grid_inside<R>(bg.grid, xf, yf, zf)) return false;
          if (loads && Gf.Bmag < R(sp_tiny)) return false;
          const v3<R> bf = !loads ? Gf.B : (is_f32<R>() ? (R(1) / Gf.Bmag) * Gf.B : Gf.B / Gf.Bmag);
          R K0f = K0, K1f = K1;
@@ -431,7 +431,7 @@ __device__ __forceinline__ int parker_step(PP P, PlanPtr Pc, LaunchPtr L, const 
          xf -= 2.0 * (double)delta * ex;
          yf -= 2.0 * (double)delta * ey;
          zf -= 2.0 * (double)delta * ez;
-         if (loads ? !grid_eval<R, false>(bg.grid, xf, yf, zf, Gb) : !grid_inside<R>(bg.grid, xf, yf, zf)) return false;
+         if (loads ? !grid_eval<R, false, V>(bg.grid, xf, yf, zf, Gb) : !grid_inside<R>(bg.grid, xf, yf, zf)) return false;
          if (loads && Gb.Bmag < R(sp_tiny)) return false;
          const v3<R> bb = !loads ? Gb.B : (is_f32<R>() ? (R(1) / Gb.Bmag) * Gb.B : Gb.B / Gb.Bmag);
          R K0b = K0, K1b = K1;
@@ -483,11 +483,11 @@ __device__ __forceinline__ int parker_step(PP P, PlanPtr Pc, LaunchPtr L, const 
          double xf = H.x + (double)delta * ex, yf = H.y + (double)delta * ey, zf = H.z + (double)delta * ez;
          const bool loads = bg.grid.fd_fields != 0;
          GridFields<R> G;
-         if (loads ? (!grid_eval<R, false>(bg.grid, xf, yf, zf, G) || G.Bmag < R(sp_tiny)) : !grid_inside<R>(bg.grid, xf, yf, zf)) return false;
+         if (loads ? (!grid_eval<R, false, V>(bg.grid, xf, yf, zf, G) || G.Bmag < R(sp_tiny)) : !grid_inside<R>(bg.grid, xf, yf, zf)) return false;
          xf -= 2.0 * (double)delta * ex;
          yf -= 2.0 * (double)delta * ey;
          zf -= 2.0 * (double)delta * ez;
-         if (loads ? (!grid_eval<R, false>(bg.grid, xf, yf, zf, G) || G.Bmag < R(sp_tiny)) : !grid_inside<R>(bg.grid, xf, yf, zf)) return false;
+         if (loads ? (!grid_eval<R, false, V>(bg.grid, xf, yf, zf, G) || G.Bmag < R(sp_tiny)) : !grid_inside<R>(bg.grid, xf, yf, zf)) return false;
          return true;
       };
       if constexpr (V == 1) {

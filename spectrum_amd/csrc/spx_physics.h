@@ -66,6 +66,22 @@ SPX_HD float rtanh(float a) { return tanhf(a); }
 template <typename R> constexpr bool is_f32() { return std::is_same<R, float>::value; }
 __device__ __forceinline__ float frsq(float x) { return __builtin_amdgcn_rsqf(x); }
 
+template <typename R> __device__ __forceinline__ void own_rounding1(R& v) { if constexpr (is_f32<R>()) asm("" : "+v"(v)); }
+template <typename R> __device__ __forceinline__ void own_rounding1(v3<R>& v)
+{
+   own_rounding1(v.x);
+   own_rounding1(v.y);
+   own_rounding1(v.z);
+}
+// A sum whose next term follows in the same basic block: the FP32 unit contracts across statements, and without
+// this it would fuse the multiply of the term already in the sum instead of the next one's, as the loop does.
+template <typename R, int N> __device__ __forceinline__ void own_rounding1(R (&v)[N])
+{
+#pragma unroll
+   for (int i = 0; i < N; i++) own_rounding1(v[i]);
+}
+template <typename... T> __device__ __forceinline__ void own_rounding(T&... v) { (own_rounding1(v), ...); }
+
 // a / c for a constant c: the FP64 kernels round it as the division does, through div_rn with the
 // reciprocal the compiler folds (correctly rounded); the FP32 unit, built with reciprocal math, keeps its
 // product by the reciprocal.  divc for the step type R, divc_d for an FP64 quantity in a kernel of step type R.
@@ -494,7 +510,7 @@ __device__ __forceinline__ bool grid_inside(GD& g, double x, double y, double z)
    return grid_locate<R>(g, x, y, z, lo, hi, dl, zone0, zl_min);
 }
 
-template <typename R, bool GRAD, typename GD>
+template <typename R, bool GRAD, int V = 0, typename GD>
 __device__ __forceinline__ bool grid_eval(GD& g, double x, double y, double z, GridFields<R>& o)
 {
    R lo[3], hi[3], dl[3];
@@ -507,8 +523,7 @@ __device__ __forceinline__ bool grid_eval(GD& g, double x, double y, double z, G
    R acc[7], dUx = R(0), dUy = R(0), dUz = R(0);
 #pragma unroll
    for (int m = 0; m < 7; m++) acc[m] = R(0);
-#pragma unroll 1
-   for (int r = 0; r < 4; r++) {
+   auto row = [&](int r) {
       const int j = r & 1, k = r >> 1;
       R v0[7], v1[7];
       grid_corner<R>(g, zone0, 2 * r, v0);
@@ -529,6 +544,20 @@ __device__ __forceinline__ bool grid_eval(GD& g, double x, double y, double z, G
             dUz = dUz + ddz * v[2];
          }
       }
+   };
+   // the few-wave form has every record of the stencil in flight at once, since no other wave hides the gather's
+   // latency (anisotropic FP64 10^4 trajectories 293 -> 281 ms); a row's sums end in it, as the loop's do
+   if constexpr (V == 1) {
+      own_rounding(acc, dUx, dUy, dUz);
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+         row(r);
+         own_rounding(acc, dUx, dUy, dUz);
+      }
+   }
+   else {
+#pragma unroll 1
+      for (int r = 0; r < 4; r++) row(r);
    }
    const R fv = R(g.f_vel), fm = R(g.f_mag);
    o.U = mk<R>(acc[0] * fv, acc[1] * fv, acc[2] * fv);
@@ -543,7 +572,7 @@ __device__ __forceinline__ bool grid_eval(GD& g, double x, double y, double z, G
 // units before the unit conversion (GetVariablesInterp1, src/server_cartesian.cc:538-560, :590-609), and
 // from the stencil's derivative weights (GetGradientsInterp1, :630-705) grad|B| and the off-diagonal
 // d B_j / d x_i that curl B needs.  gB holds (01, 02, 10, 12, 20, 21) of gradB[i][j] = d B_j / d x_i.
-template <typename R, typename GD>
+template <typename R, int V = 0, typename GD>
 __device__ __forceinline__ bool grid_eval_gc(GD& g, double x, double y, double z, v3<R>& U, v3<R>& B, R& Bmag,
                                              v3<R>& E, v3<R>& gradBmag, R gB[6], double& zl_min)
 {
@@ -557,8 +586,7 @@ __device__ __forceinline__ bool grid_eval_gc(GD& g, double x, double y, double z
    for (int m = 0; m < 3; m++) gm[m] = R(0);
 #pragma unroll
    for (int m = 0; m < 6; m++) g6[m] = R(0);
-#pragma unroll 1
-   for (int r = 0; r < 4; r++) {
+   auto row = [&](int r) {
       const int j = r & 1, k = r >> 1;
       R v0[7], v1[7];
       grid_corner<R>(g, zone0, 2 * r, v0);
@@ -581,6 +609,18 @@ __device__ __forceinline__ bool grid_eval_gc(GD& g, double x, double y, double z
          g6[4] = g6[4] + dz * v[3];   // d Bx / dz
          g6[5] = g6[5] + dz * v[4];   // d By / dz
       }
+   };
+   if constexpr (V == 1) {   // as in grid_eval
+      own_rounding(acc, gm, g6);
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+         row(r);
+         own_rounding(acc, gm, g6);
+      }
+   }
+   else {
+#pragma unroll 1
+      for (int r = 0; r < 4; r++) row(r);
    }
    const R fv = R(g.f_vel), fm = R(g.f_mag), cf = R(C_CGS / 1.0E7);
    const v3<R> Uf = mk<R>(acc[0], acc[1], acc[2]), Bf = mk<R>(acc[3], acc[4], acc[5]);
