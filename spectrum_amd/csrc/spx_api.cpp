@@ -761,6 +761,7 @@ int spx_set_background_grid(spx_sim* s, const int32_t n_blocks[3], const double 
       g.dom_min[a] = dom_min[a];
       g.dom_max[a] = dom_max[a];
       g.block_length[a] = (dom_max[a] - dom_min[a]) / (double)n_blocks[a];   // src/reader_cartesian.cc:88
+      g.block_rcp[a] = 1.0 / g.block_length[a];
       nzone *= g.nz[a];
    }
    grid_units(g);

@@ -207,7 +207,7 @@ __device__ __forceinline__ void load_hot(HotPlan<R>& h, PlanPtr P)
    SPX_HOT(eprime[0]); SPX_HOT(eprime[1]); SPX_HOT(eprime[2]); SPX_HOT(ur0); SPX_HOT(w0); SPX_HOT(hp_rad); SPX_HOT(ur0_rcp); SPX_HOT(sw_c1);
    SPX_HOT(sw_k); SPX_HOT(sw_kg); SPX_HOT(sw_r2_ok); SPX_HOT(sw_r2_min); SPX_HOT(n_shock); SPX_HOT(v_shock); SPX_HOT(compression); SPX_HOT(u1); SPX_HOT(B1);
    SPX_HOT(E0); SPX_HOT(E1); SPX_HOT(width_shock); SPX_HOT(Eu);
-   SPX_HOT(grid.nb); SPX_HOT(grid.nz); SPX_HOT(grid.dom_min); SPX_HOT(grid.dom_max); SPX_HOT(grid.block_length); SPX_HOT(grid.f_len);
+   SPX_HOT(grid.nb); SPX_HOT(grid.nz); SPX_HOT(grid.dom_min); SPX_HOT(grid.dom_max); SPX_HOT(grid.block_length); SPX_HOT(grid.block_rcp); SPX_HOT(grid.f_len);
    SPX_HOT(grid.f_vel); SPX_HOT(grid.f_mag); SPX_HOT(grid.bmag_min); SPX_HOT(grid.inner_lo); SPX_HOT(grid.inner_hi); SPX_HOT(grid.fd_fields);
    SPX_HOT(grid.z64); SPX_HOT(grid.c32);
 #undef SPX_HOT
@@ -467,7 +467,7 @@ __device__ __forceinline__ void grid_corner(GD& g, int64_t cell, int c, R v[7])
 // The position's block, its stencil's first zone and the offsets within it.  False where the
 // reference fails (outside the domain, or a stencil beyond the grid).
 template <typename R, typename GD>
-__device__ __forceinline__ bool grid_locate(GD& g, double x, double y, double z, R lo[3], R hi[3], R dl[3],
+__device__ __forceinline__ bool grid_locate(GD& g, double x, double y, double z, R lo[3], R hi[3], R dl[3], R yd[3],
                                             int64_t& zone0, double& zl_min)
 {
    const double pos[3] = {x, y, z};
@@ -475,15 +475,21 @@ __device__ __forceinline__ bool grid_locate(GD& g, double x, double y, double z,
    zl_min = 0.0;
 #pragma unroll
    for (int a = 0; a < 3; a++) {
-      const double pf = pos[a] / AU_CGS * unit_length;          // server side: position in fluid units
+      const double pf = divc_d<R>(pos[a], AU_CGS) * unit_length;   // server side: position in fluid units
       if (!(pf >= g.dom_min[a] && pf <= g.dom_max[a])) return false;
-      const int ib = (int)((pf - g.dom_min[a]) / g.block_length[a]);
+      int ib;
+      if constexpr (is_f32<R>()) ib = (int)((pf - g.dom_min[a]) / g.block_length[a]);
+      else ib = (int)div_rn(pf - g.dom_min[a], g.block_length[a], g.block_rcp[a]);
       if (ib >= g.nb[a]) return false;                          // on the upper face of the domain
       const double f0 = g.dom_min[a] + g.block_length[a] * (double)ib;
       const double face_lo = f0 * g.f_len, face_hi = (f0 + g.block_length[a]) * g.f_len;
       const double zl = (face_hi - face_lo) / (double)SPX_GRID_BLOCK;
       const double cmin = face_lo + 0.5 * zl;
-      double off = (pos[a] - cmin) / zl;
+      // FP64: the quotients by the zone length, this and the 24 derivative weights', share its correctly rounded
+      // reciprocal (with those by au and by the block length: anisotropic FP64 10^4 trajectories 279 -> 266 ms)
+      double off;
+      if constexpr (is_f32<R>()) { off = (pos[a] - cmin) / zl; yd[a] = R(0); }
+      else { yd[a] = 1.0 / zl; off = div_rn(pos[a] - cmin, zl, yd[a]); }
       int zi = (int)off;
       if (off < 0.0) zi--;
       off = off - (double)zi;
@@ -498,25 +504,32 @@ __device__ __forceinline__ bool grid_locate(GD& g, double x, double y, double z,
    return true;
 }
 
+// The derivative weight sign * a / dl of a corner: FP64 rounds the quotient as the division does.
+template <typename R> __device__ __forceinline__ R grid_dweight(R sign, R a, R dl, R yd)
+{
+   if constexpr (is_f32<R>()) return sign * a / dl;
+   else return sign * div_rn(a, dl, yd);
+}
+
 template <typename R, typename GD>
 __device__ __forceinline__ bool grid_inside(GD& g, double x, double y, double z)
 {
    // well inside the zone-centre box the answer is yes without the exact block arithmetic
    if (x > g.inner_lo[0] && x < g.inner_hi[0] && y > g.inner_lo[1] && y < g.inner_hi[1] && z > g.inner_lo[2] && z < g.inner_hi[2])
       return true;
-   R lo[3], hi[3], dl[3];
+   R lo[3], hi[3], dl[3], yd[3];
    int64_t zone0;
    double zl_min;
-   return grid_locate<R>(g, x, y, z, lo, hi, dl, zone0, zl_min);
+   return grid_locate<R>(g, x, y, z, lo, hi, dl, yd, zone0, zl_min);
 }
 
 template <typename R, bool GRAD, int V = 0, typename GD>
 __device__ __forceinline__ bool grid_eval(GD& g, double x, double y, double z, GridFields<R>& o)
 {
-   R lo[3], hi[3], dl[3];
+   R lo[3], hi[3], dl[3], yd[3];
    int64_t zone0;
    double zl_min;
-   if (!grid_locate<R>(g, x, y, z, lo, hi, dl, zone0, zl_min)) return false;
+   if (!grid_locate<R>(g, x, y, z, lo, hi, dl, yd, zone0, zl_min)) return false;
    // corners in the reference's order c = i + 2j + 4k, one row (j, k) of two x-neighbours at a time: the
    // sums start from zero as the reference's do, and a rolled loop keeps two records in flight instead
    // of eight, which leaves registers for more resident waves to hide the gather latency
@@ -538,7 +551,7 @@ __device__ __forceinline__ bool grid_eval(GD& g, double x, double y, double z, G
          for (int m = 0; m < 7; m++) acc[m] = acc[m] + w * v[m];
          if (GRAD) {   // the diagonal of grad U: d(Ux)/dx, d(Uy)/dy, d(Uz)/dz
             const R sx = i ? R(1) : R(-1), sy_ = j ? R(1) : R(-1), sz_ = k ? R(1) : R(-1);
-            const R ddx = sx * (fy * fz) / dl[0], ddy = sy_ * (fx * fz) / dl[1], ddz = sz_ * (fx * fy) / dl[2];
+            const R ddx = grid_dweight(sx, fy * fz, dl[0], yd[0]), ddy = grid_dweight(sy_, fx * fz, dl[1], yd[1]), ddz = grid_dweight(sz_, fx * fy, dl[2], yd[2]);
             dUx = dUx + ddx * v[0];
             dUy = dUy + ddy * v[1];
             dUz = dUz + ddz * v[2];
@@ -576,9 +589,9 @@ template <typename R, int V = 0, typename GD>
 __device__ __forceinline__ bool grid_eval_gc(GD& g, double x, double y, double z, v3<R>& U, v3<R>& B, R& Bmag,
                                              v3<R>& E, v3<R>& gradBmag, R gB[6], double& zl_min)
 {
-   R lo[3], hi[3], dl[3];
+   R lo[3], hi[3], dl[3], yd[3];
    int64_t zone0;
-   if (!grid_locate<R>(g, x, y, z, lo, hi, dl, zone0, zl_min)) return false;
+   if (!grid_locate<R>(g, x, y, z, lo, hi, dl, yd, zone0, zl_min)) return false;
    R acc[7], gm[3], g6[6];
 #pragma unroll
    for (int m = 0; m < 7; m++) acc[m] = R(0);
@@ -600,7 +613,7 @@ __device__ __forceinline__ bool grid_eval_gc(GD& g, double x, double y, double z
 #pragma unroll
          for (int m = 0; m < 7; m++) acc[m] = acc[m] + w * v[m];
          const R sx = i ? R(1) : R(-1), sy_ = j ? R(1) : R(-1), sz_ = k ? R(1) : R(-1);
-         const R dx = sx * (fy * fz) / dl[0], dy = sy_ * (fx * fz) / dl[1], dz = sz_ * (fx * fy) / dl[2];
+         const R dx = grid_dweight(sx, fy * fz, dl[0], yd[0]), dy = grid_dweight(sy_, fx * fz, dl[1], yd[1]), dz = grid_dweight(sz_, fx * fy, dl[2], yd[2]);
          gm[0] = gm[0] + dx * v[6]; gm[1] = gm[1] + dy * v[6]; gm[2] = gm[2] + dz * v[6];
          g6[0] = g6[0] + dx * v[4];   // d By / dx
          g6[1] = g6[1] + dx * v[5];   // d Bz / dx
@@ -643,9 +656,9 @@ template <typename R, bool GRADS, typename GD>
 __device__ __forceinline__ bool grid_eval_full(GD& g, double x, double y, double z, v3<R>& U, v3<R>& B, R& Bmag,
                                                v3<R>& E, v3<R> (&gU)[3], v3<R> (&gB)[3], v3<R>& gradBmag, double& zl_min)
 {
-   R lo[3], hi[3], dl[3];
+   R lo[3], hi[3], dl[3], yd[3];
    int64_t zone0;
-   if (!grid_locate<R>(g, x, y, z, lo, hi, dl, zone0, zl_min)) return false;
+   if (!grid_locate<R>(g, x, y, z, lo, hi, dl, yd, zone0, zl_min)) return false;
    R acc[7], gu[9], gb[9], gm[3];
 #pragma unroll
    for (int m = 0; m < 7; m++) acc[m] = R(0);
@@ -669,7 +682,7 @@ __device__ __forceinline__ bool grid_eval_full(GD& g, double x, double y, double
          for (int m = 0; m < 7; m++) acc[m] = acc[m] + w * v[m];
          if (GRADS) {
             const R sx = i ? R(1) : R(-1), sy_ = j ? R(1) : R(-1), sz_ = k ? R(1) : R(-1);
-            const R d[3] = {sx * (fy * fz) / dl[0], sy_ * (fx * fz) / dl[1], sz_ * (fx * fy) / dl[2]};
+            const R d[3] = {grid_dweight(sx, fy * fz, dl[0], yd[0]), grid_dweight(sy_, fx * fz, dl[1], yd[1]), grid_dweight(sz_, fx * fy, dl[2], yd[2])};
 #pragma unroll
             for (int a = 0; a < 3; a++) {
 #pragma unroll

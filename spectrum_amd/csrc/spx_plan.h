@@ -40,6 +40,7 @@ typedef struct {
    int32_t nb[3], nz[3];                // blocks and zones per axis
    double dom_min[3], dom_max[3];       // domain corners, fluid units (au)
    double block_length[3];              // (dom_max - dom_min) / nb, fluid units
+   double block_rcp[3];                 // 1 / block_length, correctly rounded (the FP64 kernels' quotients by it)
    double f_len, f_vel, f_mag;          // Fluid / Particle units of length, velocity, magnetic field
    double bmag_min;                     // smallest zone |B| of the grid, fluid units
    // a box in code units, a relative 1e-9 inside the first and last zone centres: a position in it has
