@@ -19,6 +19,7 @@ template <typename R>
 struct GcFields {
    v3<R> E, B, bhat, gradBmag, curlbhat;
    R Bmag, dmax;
+   R yB;               // FP64: 1 / |B|, shared by every quotient by |B| of a step
    R rg;               // the solar wind's derivative step r_g (half of SpatialData::_dr)
    v3<R> dbhatdt;      // time-dependent backgrounds (the moving smooth shock): d bhat / dt
    R dBmagdt;          // and d|B| / dt = bhat . dB/dt
@@ -48,9 +49,10 @@ __device__ __forceinline__ bool gc_fields(BD& bg, double t, double x, double y, 
       F.dmax = fmin(F.dmax, R(zl_min));
       F.rg = R(0);
       if (F.Bmag < R(sp_tiny)) return false;
-      F.bhat = F.B / F.Bmag;
+      F.yB = rcp_of(F.Bmag);
+      F.bhat = div_by(F.B, F.Bmag, F.yB);
       const v3<R> curlB = mk<R>(gB[3] - gB[5], gB[4] - gB[1], gB[0] - gB[2]);
-      F.curlbhat = (curlB - cross(F.gradBmag, F.bhat)) / F.Bmag;
+      F.curlbhat = div_by(curlB - cross(F.gradBmag, F.bhat), F.Bmag, F.yB);
       return true;
    }
    v3<R> U, B;
@@ -60,7 +62,8 @@ __device__ __forceinline__ bool gc_fields(BD& bg, double t, double x, double y, 
    F.B = B;
    F.Bmag = norm(B);
    if (F.Bmag < R(sp_tiny)) return false;
-   F.bhat = B / F.Bmag;
+   F.yB = rcp_of(F.Bmag);
+   F.bhat = div_by(B, F.Bmag, F.yB);
    if (BG == SPX_BG_UNIFORM) F.E = v3of(bg.Eu);                    // src/background_uniform.cc:58-77
    else if (BG == SPX_BG_SHOCK)                                     // src/background_shock.cc:91-111: E0 / E1 by side
       F.E = (dot(rel(bg, x, y, z), v3of(bg.n_shock)) - bg.v_shock * R(t) > R(0)) ? v3of(bg.E0) : v3of(bg.E1);
@@ -73,15 +76,15 @@ __device__ __forceinline__ bool gc_fields(BD& bg, double t, double x, double y, 
       const v3<R> g0 = f * (n.x * db), g1 = f * (n.y * db), g2 = f * (n.z * db);
       F.gradBmag = mk<R>(dot(g0, F.bhat), dot(g1, F.bhat), dot(g2, F.bhat));
       const v3<R> curlB = mk<R>(g1.z - g2.y, g2.x - g0.z, g0.y - g1.x);
-      F.curlbhat = (curlB - cross(F.gradBmag, F.bhat)) / F.Bmag;
+      F.curlbhat = div_by(curlB - cross(F.gradBmag, F.bhat), F.Bmag, F.yB);
       const v3<R> dBdt = (shock_transition_deriv(ds) * bg.v_shock / bg.width_shock) * (v3of(bg.B1) - v3of(bg.B0));
       F.dBmagdt = dot(dBdt, F.bhat);
-      F.dbhatdt = (dBdt - F.dBmagdt * F.bhat) / F.Bmag;
+      F.dbhatdt = div_by(dBdt - F.dBmagdt * F.bhat, F.Bmag, F.yB);
       F.rg = R(0);
       return true;
    }
    if (BG == SPX_BG_SOLARWIND) {
-      const R r_g = fmin(LarmorRadius(pm, F.Bmag), F.dmax);
+      const R r_g = fmin(LarmorRadius(pm, F.Bmag, F.yB), F.dmax);
       F.rg = r_g;
       v3<R> fa[3];
       fa[2] = F.bhat;
@@ -147,7 +150,7 @@ __device__ __forceinline__ bool gc_fields(BD& bg, double t, double x, double y, 
       }
       F.gradBmag = gbm;
       const v3<R> curlB = mk<R>(g12 - g21, g20 - g02, g01 - g10);
-      F.curlbhat = (curlB - cross(gbm, F.bhat)) / F.Bmag;
+      F.curlbhat = div_by(curlB - cross(gbm, F.bhat), F.Bmag, F.yB);
    }
    else {
       F.gradBmag = mk<R>(R(0), R(0), R(0));
@@ -330,16 +333,18 @@ __device__ __forceinline__ void gc_perp(DD& df, const GcFields<R>& F, const v3<R
 }
 
 // TrajectoryGuiding::DriftCoeff / ModifiedFields (src/trajectory_guiding.cc:65-146): E*, B* and the
-// guiding-centre velocity for velocity components (v_perp, 0, v_par).
+// guiding-centre velocity for velocity components (v_perp, 0, v_par).  Bpar = B* . bhat and its FP64 reciprocal.
 template <typename R, int BG>
-__device__ __forceinline__ void gc_drift(const GcFields<R>& F, v3<R> vel, R pp, R pl, v3<R>& drift, v3<R>& Es, v3<R>& Bs)
+__device__ __forceinline__ void gc_drift(const GcFields<R>& F, v3<R> vel, R pp, R pl, v3<R>& drift, v3<R>& Es, v3<R>& Bs, R& Bpar, R& yBpar)
 {
-   const R rL = LarmorRadius(pp, F.Bmag), rR = LarmorRadius(pl, F.Bmag);
+   const R rL = LarmorRadius(pp, F.Bmag, F.yB), rR = LarmorRadius(pl, F.Bmag, F.yB);
    if (BG == SPX_BG_SMOOTHSHOCK)   // the time-dependent term -r_R |B| (d bhat/dt) / c of E*
       Es = (F.E - ((rR * F.Bmag) * F.dbhatdt) / R(c_code)) - ((rL * vel.x) * F.gradBmag) / (R(2) * R(c_code));
    else Es = F.E - ((rL * vel.x) * F.gradBmag) / (R(2) * R(c_code));
    Bs = F.B + (rR * F.Bmag) * F.curlbhat;
-   drift = (vel.z * Bs + R(c_code) * cross(Es, F.bhat)) / dot(Bs, F.bhat);
+   Bpar = dot(Bs, F.bhat);
+   yBpar = rcp_of(Bpar);
+   drift = div_by(vel.z * Bs + R(c_code) * cross(Es, F.bhat), Bpar, yBpar);
 }
 
 // Particle velocity for a guiding-centre momentum (p_perp, 0, p_par) (common/physics.hh:290-297).
@@ -493,7 +498,8 @@ __device__ __forceinline__ int gc_step(PP P, PlanPtr Pc, LaunchPtr L, const spx_
    R Dmumu = R(0), Vmu = R(0);
    if (pa_step) gc_dmumu<R, XD>(df, pmag, H.F.Bmag, mu, H.x, H.y, H.z, Dmumu, Vmu);
    v3<R> drift, Es, Bs;
-   gc_drift<R, BG>(H.F, vel, pp, pl, drift, Es, Bs);
+   R Bpar, yBpar;
+   gc_drift<R, BG>(H.F, vel, pp, pl, drift, Es, Bs, Bpar, yBpar);
    // PhysicalStep: TrajectoryGuiding's (src/trajectory_guiding.cc:96-100), GuidingDiff's with V_perp and
    // D_perp (src/trajectory_guiding_diff.cc:306-314), GuidingScatt's pitch-angle limits (:255-262)
    R dtp = R(0.5) * H.F.dmax / ((perp_step ? norm(drift + Vperp) : norm(drift)) + R(0.5) * norm(vel));
@@ -551,10 +557,10 @@ __device__ __forceinline__ int gc_step(PP P, PlanPtr Pc, LaunchPtr L, const spx_
       vel = gc_vel(pp, pl);
    }
    // Slopes with the scattered momentum
-   gc_drift<R, BG>(H.F, vel, pp, pl, drift, Es, Bs);
-   const R slope_pp = (BG == SPX_BG_SMOOTHSHOCK) ? R(0.5) * pp / H.F.Bmag * (H.F.dBmagdt + dot(drift, H.F.gradBmag))
-                                                 : R(0.5) * pp / H.F.Bmag * dot(drift, H.F.gradBmag);
-   const R slope_pl = R(sp_charge) * dot(Es, Bs) / dot(Bs, H.F.bhat);
+   gc_drift<R, BG>(H.F, vel, pp, pl, drift, Es, Bs, Bpar, yBpar);
+   const R slope_pp = (BG == SPX_BG_SMOOTHSHOCK) ? div_by(R(0.5) * pp, H.F.Bmag, H.F.yB) * (H.F.dBmagdt + dot(drift, H.F.gradBmag))
+                                                 : div_by(R(0.5) * pp, H.F.Bmag, H.F.yB) * dot(drift, H.F.gradBmag);
+   const R slope_pl = div_by(R(sp_charge) * dot(Es, Bs), Bpar, yBpar);
    pmag = rsqrt_(sqr(pp) + sqr(pl));
    v3<R> slope_pos = drift;
    v3<R> dr = mk<R>(R(0), R(0), R(0));

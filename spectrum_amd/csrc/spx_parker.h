@@ -25,6 +25,7 @@ template <typename R>
 struct PkFields {
    v3<R> U, bhat;
    R Bmag, divU, dmax;
+   R yB;             // FP64: 1 / |B|
    v3<R> fa0, fa1;   // SolarWind: the field-aligned frame of bhat (second unit vector, bhat x it), reused by the step
 };
 
@@ -44,8 +45,9 @@ __device__ __forceinline__ bool parker_fields(BD& bg, double t, double x, double
       F.U = G.U;
       F.Bmag = G.Bmag;
       if (F.Bmag < R(sp_tiny)) return false;
+      F.yB = rcp_of(F.Bmag);
       if constexpr (is_f32<R>()) F.bhat = (R(1) / F.Bmag) * G.B;
-      else F.bhat = G.B / F.Bmag;
+      else F.bhat = div_by(G.B, F.Bmag, F.yB);
       F.divU = G.divU;
       return true;
    }
@@ -62,10 +64,11 @@ __device__ __forceinline__ bool parker_fields(BD& bg, double t, double x, double
    else {
       F.Bmag = norm(B);
       if (F.Bmag < R(sp_tiny)) return false;
-      F.bhat = B / F.Bmag;
+      F.yB = rcp_of(F.Bmag);
+      F.bhat = div_by(B, F.Bmag, F.yB);
    }
    if (BG == SPX_BG_SOLARWIND) {
-      const R r_g = fmin(LarmorRadius(p, F.Bmag), F.dmax);
+      const R r_g = fmin(LarmorRadius(p, F.Bmag, F.yB), F.dmax);
       v3<R> fa[3];
       fa[2] = F.bhat;
       fa[0] = second_unit(F.bhat);
@@ -354,7 +357,7 @@ __device__ __forceinline__ int parker_step(PP P, PlanPtr Pc, LaunchPtr L, const 
       else if (df.kind == SPX_DF_SOQLT) { km2 = kappa_mom_soqlt(df, p, 0, false); km3 = kappa_mom_soqlt(df, p, 0, true); }
    }
    parker_kappa<R, BG, DF>(bg, df, km, km2, km3, H.F.Bmag, H.x, H.y, H.z, H.F.U, K0, K1);
-   const R delta = fmin(LarmorRadius(p, H.F.Bmag), H.F.dmax);
+   const R delta = fmin(LarmorRadius(p, H.F.Bmag, H.F.yB), H.F.dmax);
    const R hdi = is_f32<R>() ? R(0.5) / delta : R(0);
    const double ydel = is_f32<R>() ? 0.0 : 1.0 / (double)delta;   // FP64: the stencil's nine quotients by delta share it
    v3<R> divK = mk<R>(R(0), R(0), R(0));

@@ -120,6 +120,27 @@ template <typename R> SPX_HD R EnrKin(R p) { return EnrTot(p) - R(sp_mass * (c_c
 template <typename R> SPX_HD R VelP(R p) { return p * R(c_code * c_code) / EnrTot(p); }
 template <typename R> SPX_HD R Rigidity(R p) { return p * R(c_code) / R(fabs(sp_charge)); }
 template <typename R> SPX_HD R LarmorRadius(R p, R B) { return p * R(c_code) / (R(fabs(sp_charge)) * B); }
+// Quotients by a length b whose reciprocal yb = 1 / b the caller keeps (FP64, rounded as the division; the FP32 unit divides).
+template <typename R> SPX_HD R rcp_of(R b)
+{
+   if constexpr (is_f32<R>()) return R(0);
+   else return R(1) / b;
+}
+template <typename R> SPX_HD R div_by(R a, R b, R yb)
+{
+   if constexpr (is_f32<R>()) return a / b;
+   else return div_rn(a, b, yb);
+}
+template <typename R> SPX_HD v3<R> div_by(v3<R> a, R b, R yb)
+{
+   if constexpr (is_f32<R>()) return a / b;
+   else return mk<R>(div_rn(a.x, b, yb), div_rn(a.y, b, yb), div_rn(a.z, b, yb));
+}
+template <typename R> SPX_HD R LarmorRadius(R p, R B, R yB)   // the charge is 1: q B == B
+{
+   if constexpr (is_f32<R>()) return LarmorRadius(p, B);
+   else return div_rn(p * R(c_code), B, yB);
+}
 template <typename R> SPX_HD R RelFactor(R v) { return R(1) / rsqrt_(R(1) - sqr(v / R(c_code))); }
 template <typename R> SPX_HD R CyclotronFrequency(R v, R B) { return R(sp_charge) * B / (RelFactor(v) * R(sp_mass) * R(c_code)); }
 // Particle::Mom (common/physics.hh:262-266)
