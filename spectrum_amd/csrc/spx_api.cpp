@@ -932,9 +932,10 @@ int spx_finish(spx_sim* s, spx_traj_record* records, spx_run_stats* st)
    s->pool.step_ms = s->pool.service_ms = 0.0;
    double kms = 0.0;
    int launches = 0;
-   // Every launch advances each live slot by min(steps_per_launch, 100) steps or more (Pool::round); a trajectory
-   // needs at most max_attempts * (max_steps + 1) steps, so this bound is never reached by a healthy run.
-   const double guard = 64.0 + (double)s->plan.max_attempts * ((double)s->plan.max_steps + 1.0) / std::min(s->steps_per_launch, 100) *
+   // Every second launch or more advances a live slot, by min(steps_per_launch, 100) steps or more (Pool::round,
+   // step_window); a trajectory needs at most max_attempts * (max_steps + 1) steps, so this bound is never reached by a
+   // healthy run.
+   const double guard = 64.0 + 2.0 * (double)s->plan.max_attempts * ((double)s->plan.max_steps + 1.0) / std::min(s->steps_per_launch, 100) *
                                    std::max(1.0, (double)s->run_n / (double)s->pool.n_lanes + 1.0);
    while (true) {
       RunCtl ctl;
@@ -1380,7 +1381,7 @@ int spx_main_loop(spx_sim* s, const spx_rng* rng, spx_run_stats* st)
       if (rc) return rc;
       const auto w0 = std::chrono::steady_clock::now();
       s->pool.step_ms = s->pool.service_ms = 0.0;
-      const double guard = 64.0 + (double)s->plan.max_attempts * ((double)s->plan.max_steps + 1.0) / std::min(s->steps_per_launch, 100) *
+      const double guard = 64.0 + 2.0 * (double)s->plan.max_attempts * ((double)s->plan.max_steps + 1.0) / std::min(s->steps_per_launch, 100) *
                                       std::max(1.0, (double)n_total / (double)s->pool.n_lanes + 1.0);
       int percentage_done = 0, launches = 0;
       while (true) {

@@ -608,13 +608,13 @@ __device__ __forceinline__ int gc_step(PP P, PlanPtr Pc, LaunchPtr L, const spx_
 #endif
 
 template <typename R, int BG, bool XD, int V>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(V == 1 ? 1 : SPX_GC_WAVES))) void gc_step_kernel(const Launch* __restrict__ Lg, int32_t packed, int32_t n_steps)
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(V == 1 ? 1 : SPX_GC_WAVES))) void gc_step_kernel(const Launch* __restrict__ Lg, int32_t packed, int32_t n_steps, uint32_t first_slot, uint32_t span)
 {
    const LaunchPtr Lp = (LaunchPtr)Lg;
    __shared__ ColdLDS C;
    const int tid = threadIdx.x;
    __shared__ RingLDS<R, V> ring;
-   const int32_t place = slot_of<V>(Lp, packed);
+   const int32_t place = slot_of<V>(Lp, packed, first_slot, span);
    const int32_t place0 = __builtin_amdgcn_readfirstlane(place);
    if (place0 < 0) return;
    const uint64_t slot = place < 0 ? (uint64_t)place0 : (uint64_t)place;
@@ -718,8 +718,11 @@ static hipError_t launch_gc_bg(const LaunchShape& S, const Launch* d_launch, hip
       }
    }
    constexpr int V = (M == LAUNCH_FEW) ? 1 : 0;
-   if constexpr (M != LAUNCH_SERVICE)
-      hipLaunchKernelGGL((gc_step_kernel<R, BG, XD, V>), dim3(step_grid<V>(S)), dim3(BLOCK), 0, st, d_launch, S.packed, S.n_steps);
+   if constexpr (M != LAUNCH_SERVICE) {
+      static const uint64_t resident = V == 1 ? 0 : resident_waves(gc_step_kernel<R, BG, XD, V>);
+      const StepWindow w = step_window<V>(S, resident);
+      hipLaunchKernelGGL((gc_step_kernel<R, BG, XD, V>), dim3(w.grid), dim3(BLOCK), 0, st, d_launch, S.packed, S.n_steps, w.first, w.span);
+   }
    return hipGetLastError();
 }
 

@@ -86,6 +86,7 @@ struct LaunchShape {
    // The step kernel takes the running slots from a list that packs them into full waves, a query's in consecutive
    // places from a wave boundary; -1: the slots in place.  0 or 1 picks the set of n_running the launch uses.
    int32_t packed = -1;
+   int64_t turn = -1;                   // launches of the run so far, where a launch may leave slots for the next (step_window)
    uint64_t list_span = 0;              // list places the step kernel covers (whole waves): at least those in use
 };
 

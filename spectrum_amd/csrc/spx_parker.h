@@ -659,13 +659,13 @@ __device__ __forceinline__ int parker_step(PP P, PlanPtr Pc, LaunchPtr L, const 
 }
 
 template <typename R, int BG, int FWD, int TT, int DF, int V>
-__device__ __forceinline__ void parker_step_body(const Launch* __restrict__ Lg, int32_t packed, int32_t n_steps)
+__device__ __forceinline__ void parker_step_body(const Launch* __restrict__ Lg, int32_t packed, int32_t n_steps, uint32_t first_slot, uint32_t span)
 {
    const LaunchPtr Lp = (LaunchPtr)Lg;
    __shared__ ColdLDS C;
    const int tid = threadIdx.x;
    __shared__ RingLDS<R, V> ring;
-   const int32_t place = slot_of<V>(Lp, packed);
+   const int32_t place = slot_of<V>(Lp, packed, first_slot, span);
    const int32_t place0 = __builtin_amdgcn_readfirstlane(place);
    if (place0 < 0) return;
    const uint64_t slot = place < 0 ? (uint64_t)place0 : (uint64_t)place;
@@ -783,9 +783,9 @@ constexpr int pk_waves()
 }
 template <typename R, int BG, int FWD, int TT, int DF, int V>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(V == 1 ? 1 : pk_waves<R, BG, TT, DF>())))
-void parker_step_kernel(const Launch* __restrict__ Lg, int32_t packed, int32_t n_steps)
+void parker_step_kernel(const Launch* __restrict__ Lg, int32_t packed, int32_t n_steps, uint32_t first_slot, uint32_t span)
 {
-   parker_step_body<R, BG, FWD, TT, DF, V>(Lg, packed, n_steps);
+   parker_step_body<R, BG, FWD, TT, DF, V>(Lg, packed, n_steps, first_slot, span);
 }
 
 // The gridded background's step kernel waits on gathers: its V = 0 form asks the compiler for room for
@@ -794,9 +794,9 @@ void parker_step_kernel(const Launch* __restrict__ Lg, int32_t packed, int32_t n
 #define SPX_GRID_WAVES 2
 #endif
 template <typename R, int FWD, int TT, int V>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(V == 1 ? 1 : SPX_GRID_WAVES))) void parker_grid_step_kernel(const Launch* __restrict__ Lg, int32_t packed, int32_t n_steps)
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(V == 1 ? 1 : SPX_GRID_WAVES))) void parker_grid_step_kernel(const Launch* __restrict__ Lg, int32_t packed, int32_t n_steps, uint32_t first_slot, uint32_t span)
 {
-   parker_step_body<R, SPX_BG_GRID, FWD, TT, 0, V>(Lg, packed, n_steps);
+   parker_step_body<R, SPX_BG_GRID, FWD, TT, 0, V>(Lg, packed, n_steps, first_slot, span);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -818,9 +818,13 @@ static hipError_t launch_parker(const LaunchShape& S, const Launch* d_launch, hi
    }
    if constexpr (M != LAUNCH_SERVICE) {
       constexpr int V = (M == LAUNCH_FEW) ? 1 : 0;
-      const unsigned sg = step_grid<V>(S);
-      if constexpr (BG == SPX_BG_GRID) hipLaunchKernelGGL((parker_grid_step_kernel<R, FWD, TT, V>), dim3(sg), dim3(BLOCK), 0, st, d_launch, S.packed, S.n_steps);
-      else hipLaunchKernelGGL((parker_step_kernel<R, BG, FWD, TT, DF, V>), dim3(sg), dim3(BLOCK), 0, st, d_launch, S.packed, S.n_steps);
+      auto* kernel = [] {
+         if constexpr (BG == SPX_BG_GRID) return &parker_grid_step_kernel<R, FWD, TT, V>;
+         else return &parker_step_kernel<R, BG, FWD, TT, DF, V>;
+      }();
+      static const uint64_t resident = V == 1 ? 0 : resident_waves(kernel);
+      const StepWindow w = step_window<V>(S, resident);
+      hipLaunchKernelGGL(kernel, dim3(w.grid), dim3(BLOCK), 0, st, d_launch, S.packed, S.n_steps, w.first, w.span);
    }
    return hipGetLastError();
 }

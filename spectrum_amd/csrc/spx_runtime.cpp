@@ -327,6 +327,7 @@ hipError_t Pool::launch(int n, const LaunchShape& S0, float* ms_out)
          TRY(hipEventRecord(tev[2 * i], stream));
          take_turn(S);
          TRY(launch_transport(sig, S, d_launch.p, precision, stream, tev[2 * i + 1]));
+         if (S.turn >= 0) S.turn++;
       }
       launches += n;
    }
@@ -363,7 +364,9 @@ hipError_t Pool::round(uint64_t live, bool claimed, double& ms_total, int& n_lau
       n = std::max(1, std::min(8, (int)(want / steps)));
    }
    float ms = 0.f;
-   TRY(launch(n, shape(live, claimed, steps), &ms));
+   LaunchShape S = shape(live, claimed, steps);
+   S.turn = launches;
+   TRY(launch(n, S, &ms));
    ms_per_step = graph_launches == 0 ? (double)ms / ((double)n * steps) : 0.0;
    ms_total += ms;
    n_launches += n;
