@@ -194,7 +194,7 @@ __device__ __noinline__ void wnlt_k(DD& df, bool comp2, double x, double y, doub
 {
    R k_min = df.k_min, A2A = df.A2A, A2T = df.A2T, A2L = df.A2L;
    if (df.kind == SPX_DF_WNLT_RAMP) {
-      const double r0 = norm(mk<double>(x, y, z));
+      const double r0 = norm_d<R>(x, y, z);
       const R z0 = R(sqrt(0.5 * r0 * (r0 + z)));
       if (z0 > df.z_sheath) { k_min = df.k_min_ref; A2A = df.A2A_ref; A2T = df.A2T_ref; A2L = df.A2L_ref; }
       else {
@@ -241,7 +241,7 @@ __device__ __forceinline__ R gc_kperp(DD& df, R pmag, R mu, R Bmag, double x, do
          return K0;
       }
       if (df.kind == SPX_DF_SOQLT) {   // :1053-1072; `outer` is region[Bmix_idx] < 0, the radius is this point's
-         const bool reduced = outer && norm(mk<double>(x, y, z)) < (double)df.r_lim_red;
+         const bool reduced = outer && norm_d<R>(x, y, z) < (double)df.r_lim_red;
          R K0 = kappa_mom_soqlt(df, pmag, 0, reduced) * (df.B0 / Bmag);
          K0 = K0 / df.sc_den;
          return K0;

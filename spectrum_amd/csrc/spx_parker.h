@@ -160,7 +160,8 @@ __device__ __forceinline__ bool lism_outer(BD& bg, DD& df, double x, double y, d
 // DiffusionBase::GetComponent for components 0 and 1 at a position.  DF is the diffusion class when it
 // is known at compile time (0 = any, dispatched at run time); km2 is the LISM factor of the region models,
 // or with km3 the two perpendicular factors of the empirical SOQLT model (lam_perp, lam_perp kap_rat_red).
-template <typename R, int BG, int DF, typename BD, typename DD>
+// CENTRE: at the step's own position (norm_d).
+template <typename R, int BG, int DF, bool CENTRE = false, typename BD, typename DD>
 __device__ __forceinline__ void parker_kappa(BD& bg, DD& df, R km, R km2, R km3, R Bmag,
                                              double x, double y, double z, v3<R> U, R& K0, R& K1)
 {
@@ -179,7 +180,7 @@ __device__ __forceinline__ void parker_kappa(BD& bg, DD& df, R km, R km2, R km3,
    }
    if (df.kind == SPX_DF_SOQLT) {                                         // :1053-1072
       // the reduced perpendicular path inside r_lim_red where region[Bmix_idx] < 0 (lism_outer reads it)
-      const bool reduced = lism_outer<R, BG>(bg, df, x, y, z) && norm(mk<double>(x, y, z)) < (double)df.r_lim_red;
+      const bool reduced = lism_outer<R, BG>(bg, df, x, y, z) && norm_d<R, CENTRE>(x, y, z) < (double)df.r_lim_red;
       const R bf = df.B0 / Bmag;
       K1 = km * bf;
       K1 = K1 / df.sc_den;
@@ -188,7 +189,7 @@ __device__ __forceinline__ void parker_kappa(BD& bg, DD& df, R km, R km2, R km3,
       return;
    }
    R r = R(0), Umag = R(0);
-   if (df.kind == SPX_DF_KINRAD) r = R(norm(mk<double>(x, y, z)));
+   if (df.kind == SPX_DF_KINRAD) r = R(norm_d<R, CENTRE>(x, y, z));
    if (df.kind == SPX_DF_FLOWMOM || (df.kind == SPX_DF_KINRAD && df.stream_dep_idx != 0)) Umag = norm(U);
    kappa01(df, km, Bmag, r, Umag, K0, K1);
 }
@@ -356,7 +357,7 @@ __device__ __forceinline__ int parker_step(PP P, PlanPtr Pc, LaunchPtr L, const 
       if ((df.kind == SPX_DF_STRAUSS || df.kind == SPX_DF_POTGIETER) && df.region_idx >= 0) km2 = kappa_mom_region(df, p, true);
       else if (df.kind == SPX_DF_SOQLT) { km2 = kappa_mom_soqlt(df, p, 0, false); km3 = kappa_mom_soqlt(df, p, 0, true); }
    }
-   parker_kappa<R, BG, DF>(bg, df, km, km2, km3, H.F.Bmag, H.x, H.y, H.z, H.F.U, K0, K1);
+   parker_kappa<R, BG, DF, true>(bg, df, km, km2, km3, H.F.Bmag, H.x, H.y, H.z, H.F.U, K0, K1);
    const R delta = fmin(LarmorRadius(p, H.F.Bmag, H.F.yB), H.F.dmax);
    const R hdi = is_f32<R>() ? R(0.5) / delta : R(0);
    const double ydel = is_f32<R>() ? 0.0 : 1.0 / (double)delta;   // FP64: the stencil's nine quotients by delta share it
@@ -379,12 +380,12 @@ __device__ __forceinline__ int parker_step(PP P, PlanPtr Pc, LaunchPtr L, const 
          double xf = H.x + (double)delta * ex, yf = H.y + (double)delta * ey, zf = H.z + (double)delta * ez;
          bool ok = true;
          if constexpr (BG == SPX_BG_GRID) ok = grid_inside<R>(bg.grid, xf, yf, zf);
-         const R rf = R(norm(mk<double>(xf, yf, zf))) / df.r0;
+         const R rf = R(norm_d<R>(xf, yf, zf)) / df.r0;
          xf -= 2.0 * (double)delta * ex;
          yf -= 2.0 * (double)delta * ey;
          zf -= 2.0 * (double)delta * ez;
          if constexpr (BG == SPX_BG_GRID) ok = ok && grid_inside<R>(bg.grid, xf, yf, zf);
-         const R rb = R(norm(mk<double>(xf, yf, zf))) / df.r0;
+         const R rb = R(norm_d<R>(xf, yf, zf)) / df.r0;
          R Kf, Kb;
          if (square) { Kf = km * (rf * rf); Kb = km * (rb * rb); }
          else { Kf = km * rpow(rf, df.pow_law_r); Kb = km * rpow(rb, df.pow_law_r); }

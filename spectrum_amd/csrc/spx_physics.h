@@ -102,6 +102,16 @@ template <typename R> SPX_HD double sqrt_d(double x)
    if constexpr (is_f32<R>()) return sqrt(x);
    else return sqrt_rn(x);
 }
+// |x| of an FP64 position in a kernel of step type R.  The FP32 units contract a sum of products into either
+// multiply-add, by how often each product is used in its basic block, so the sum of squares would round differently from
+// one form of a kernel to the next; both pairings are written out: a step's own position (CENTRE) rounds x^2 and fuses
+// y^2, any other point the other way about, as the one-lane kernels with the general stencil have them.
+template <typename R, bool CENTRE = false> __device__ __forceinline__ double norm_d(double x, double y, double z)
+{
+   if constexpr (!is_f32<R>()) return norm(mk<double>(x, y, z));
+   else if constexpr (CENTRE) return sqrt_rn(__builtin_fma(z, z, __builtin_fma(y, y, x * x)));
+   else return sqrt_rn(__builtin_fma(z, z, __builtin_fma(x, x, y * y)));
+}
 
 // Compensated (Kahan) addition of an increment to an FP64 sum, for the FP32-step kernels: c carries what
 // the rounding of s dropped (less than an ulp of s, so FP32 holds it to 24 bits) into the next addition.
