@@ -32,9 +32,6 @@ __device__ __forceinline__ spx_rng_desc load_rng(QueryPtr Q)
    return r;
 }
 
-// Slot states
-enum { SLOT_IDLE = 0, SLOT_RUN = 1, SLOT_START = 2, SLOT_EVENT = 3, SLOT_DONE = 4, SLOT_DISCARD = 5 };
-
 // One wave per workgroup: no lane works with another wave's, and single waves spread over the SIMDs of every CU and
 // refill one at a time where a workgroup of four waits for the last.  With the launches bounded to the slots a run can
 // fill (Pool::span): 20000 FP64 shock trajectories 1554 -> 1355 ms, 30000 of kappa ~ T r^2 128 -> 112 ms, 100000 FP64
@@ -867,7 +864,7 @@ __device__ __forceinline__ void service_slot(LaunchPtr L, int32_t packed, StartF
       const uint64_t mask = __ballot(st == SLOT_RUN);
       if (mask != 0) {
          uint32_t base = 0;
-         if (lane_id() == 0) base = atomicAdd(&L->n_running[packed * L->n_queries + q], (uint32_t)__popcll(mask));
+         if (lane_id() == 0) base = atomicAdd(&L->n_running[(int64_t)packed * L->n_queries + q], (uint32_t)__popcll(mask));
          base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
          if (st == SLOT_RUN) L->rank[slot] = (int32_t)(base + (uint32_t)__popcll(mask & lanes_below()));
       }

@@ -78,6 +78,32 @@ struct Launch {
    int32_t n_queries, pad_;             // size of the query table
 };
 
+// Slot states
+enum { SLOT_IDLE = 0, SLOT_RUN = 1, SLOT_START = 2, SLOT_EVENT = 3, SLOT_DONE = 4, SLOT_DISCARD = 5 };
+
+// Thread i of n_threads of the packing pass of a launch, one per slot of the span and per list place at least: a running
+// slot goes to its query's part of the list, a place that no slot takes gets -1, and the other set of counts is cleared
+// for the next packed launch, all of it however large the query table is.  The parts follow the admission order, each
+// from a wave boundary.
+template <typename LP>
+__host__ __device__ __forceinline__ void pack_place(LP L, int32_t packed, uint64_t span, uint64_t list_span, uint64_t i, uint64_t n_threads)
+{
+   const uint32_t* n_running = L->n_running + (int64_t)packed * L->n_queries;
+   uint32_t* other = L->n_running + (int64_t)(1 - packed) * L->n_queries;
+   const int32_t q = i < span && L->active[i] == SLOT_RUN ? L->slot_q[i] : -1;
+   uint64_t start = 0;
+   bool taken = false;
+   for (int k = 0; k < L->n_queue; k++) {
+      const int32_t c = L->queue[k];
+      const uint32_t n = n_running[c];
+      if (c == q) L->list[start + (uint64_t)L->rank[i]] = (int32_t)i;
+      taken = taken || (i >= start && i < start + n);
+      start += (n + 63u) & ~63u;
+   }
+   if (i < list_span && !taken) L->list[i] = -1;
+   for (uint64_t c = i; c < (uint64_t)L->n_queries; c += n_threads) other[c] = 0u;
+}
+
 // What one engine launch covers.
 struct LaunchShape {
    uint64_t span = 0;                   // slots the service kernel covers: the first `span`, whole blocks

@@ -35,31 +35,14 @@ hipError_t grid_expand_cells(const double* zones, const int32_t nz[3], float* c3
    return hipGetLastError();
 }
 
-// One thread per slot and per list place: a running slot goes to its query's part of the list, a place that no slot
-// takes gets -1, and the other set of counts is cleared for the next packed launch.  The parts follow the admission
-// order, each from a wave boundary.
 __global__ __launch_bounds__(256) void pack_running_kernel(const Launch* __restrict__ Lg, int32_t packed, uint64_t span, uint64_t list_span)
 {
-   const LaunchPtr L = (LaunchPtr)Lg;
-   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-   const uint32_t* n_running = L->n_running + packed * L->n_queries;
-   const int32_t q = i < span && L->active[i] == SLOT_RUN ? L->slot_q[i] : -1;
-   uint64_t start = 0;
-   bool taken = false;
-   for (int k = 0; k < L->n_queue; k++) {
-      const int32_t c = L->queue[k];
-      const uint32_t n = n_running[c];
-      if (c == q) L->list[start + (uint64_t)L->rank[i]] = (int32_t)i;
-      taken = taken || (i >= start && i < start + n);
-      start += (n + 63u) & ~63u;
-   }
-   if (i < list_span && !taken) L->list[i] = -1;
-   if (i < (uint64_t)L->n_queries) L->n_running[(1 - packed) * L->n_queries + (int32_t)i] = 0u;
+   pack_place((LaunchPtr)Lg, packed, span, list_span, (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, (uint64_t)gridDim.x * blockDim.x);
 }
 
 hipError_t pack_running(const LaunchShape& S, const Launch* d_launch, hipStream_t st)
 {
-   const uint64_t n = S.span > S.list_span ? S.span : S.list_span;   // at least a block, which is more than the query table
+   const uint64_t n = S.span > S.list_span ? S.span : S.list_span;
    hipLaunchKernelGGL(pack_running_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, d_launch, S.packed, S.span, S.list_span);
    return hipGetLastError();
 }
