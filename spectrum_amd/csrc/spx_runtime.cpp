@@ -240,7 +240,8 @@ hipError_t Pool::set_query(int q, const QueryDesc& d)
 hipError_t Pool::push_queue(int q, uint64_t n_traj)
 {
    if (host_queue.empty()) span = 0;   // every slot is idle
-   const uint64_t want = n_traj < n_lanes ? (n_traj + 255) / 256 * 256 : n_lanes;
+   // a run of no trajectories still launches, over one block
+   const uint64_t want = n_traj < n_lanes ? (std::max<uint64_t>(n_traj, 1) + 255) / 256 * 256 : n_lanes;
    span = std::min(n_lanes, span + want);
    host_queue.push_back(q);
    return upload_launch();
