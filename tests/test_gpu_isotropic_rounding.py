@@ -52,6 +52,24 @@ def test_isotropic_path_is_the_general_stencil(exponent, gridded, precision):
         same(rec, ref, f"graph {graph}")
 
 
+@pytest.mark.parametrize("precision", [E.PREC_FP64, E.PREC_MIXED])
+@pytest.mark.parametrize("exponent", [2.0, 0.5])
+def test_guard_on_the_stencil_length(exponent, precision):
+    """The isotropic path is refused where the stencil's half length h exceeds |x| / 2.  In a field this weak the Larmor
+    radius is several au and more, so h = min(0.6 |x|, 1 au): refused below 2 au, taken above."""
+    sw = cf.solarwind(B_nT_1au=1.0e-4, dmax0=cf.one_au, dmax_fraction=0.6)
+    n = 4097
+    st, ref = run(setup(exponent, general=True, sw=sw), n, precision, graph_launches=1)
+    r0 = np.linalg.norm(ref["pos0"], axis=1) / cf.one_au
+    r1 = np.linalg.norm(ref["pos"], axis=1) / cf.one_au
+    p = ref["mom0"][:, 0].min()
+    larmor = p * cf.c_code / (1.0e-13 * 1.0e4 / cf.unit_magnetic) / cf.one_au   # at 1 au; it grows with the distance squared
+    assert larmor * 0.3 ** 2 > 1.0 and (r0 < 2.0).all() and (r1 > 4.0).sum() > 100   # these cross 2 au
+    for graph in (1, 0):
+        _, rec = run(setup(exponent, sw=sw), n, precision, graph_launches=graph)
+        same(rec, ref, f"graph {graph}")
+
+
 @pytest.mark.parametrize("gridded", [False, True])
 def test_mixed_long(gridded):
     """Several 10^9 steps: the general stencil and the isotropic path with one lane, and with four in runs that fit
