@@ -657,7 +657,10 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(V == 1 ? 
    int exc = 0;
    unsigned long long steps_here = 0;
    HotPlan<R> hot;
-   if constexpr (V == 1 && !is_f32<R>()) load_hot(hot, P);
+   // the XD models hand the descriptor to a function of its own (wnlt_k): a copy of the plan would live in memory per
+   // lane (1600 B, its uniform bounds and branches read by every lane) instead of in registers
+   constexpr bool HOT = V == 1 && !is_f32<R>() && !XD;
+   if constexpr (HOT) load_hot(hot, P);
    for (int it = 0; it < n_steps; it++) {
       if (__ballot(st == SLOT_RUN) == 0) break;
       if (st != SLOT_RUN) continue;
@@ -667,7 +670,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(V == 1 ? 
       asm volatile("" : "+s"(Li));
       int bflags = 0;
       int e;
-      if constexpr (V == 1 && !is_f32<R>()) {
+      if constexpr (HOT) {
          const HotPlan<R>* h = &hot;
          e = gc_step<R, BG, XD, V>(h, Pi, Li, rng, first, slot, H, C, tid, bflags);
       }
