@@ -1,5 +1,5 @@
-"""What the compiler gave the four-lane FP64 step kernels, from the code object in the built library: the plan that they
-keep in registers must not end up in memory per lane."""
+"""What the compiler gave the step kernels, from the code object in the built library: the plan that the four-lane FP64
+kernels keep in registers must not end up in memory per lane, nor a step's state of the gridded FP32 kernels."""
 import os
 import re
 import shutil
@@ -51,3 +51,14 @@ def test_four_lane_kernels_keep_the_plan_in_registers(tmp_path):
     assert len(quad) > 40, sorted(of)[:5]
     # the arguments and results of a called function at most; the plan would take more than a kilobyte
     assert max(quad.values()) <= 64, {k: v for k, v in quad.items() if v > 64}
+
+
+def test_gridded_fp32_kernels_hold_a_step_in_registers(tmp_path):
+    if not READELF or not os.path.exists(E.LIB_PATH):
+        pytest.skip("llvm-readelf or the built library missing")
+    of = scratch(tmp_path)
+    one_lane = {k: v for k, v in of.items() if re.search(r"parker_grid_step_kernelIf\w*Li0EEEv", k)}
+    assert len(one_lane) == 6
+    for k, v in one_lane.items():
+        # what is spilled once around the step loop; the kernels with a source keep four more values per trajectory
+        assert v <= (92 if re.search(r"IfLi[01]ELi1E", k) else 16), (k, v)
