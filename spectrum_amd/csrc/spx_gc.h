@@ -656,7 +656,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(V == 1 ? 
    int st = run ? SLOT_RUN : SLOT_IDLE;
    int exc = 0;
    unsigned long long steps_here = 0;
-   HotPlan<R> hot;
+   HotPlan hot;
    // the XD models hand the descriptor to a function of its own (wnlt_k): a copy of the plan would live in memory per
    // lane (1600 B, its uniform bounds and branches read by every lane) instead of in registers
    constexpr bool HOT = V == 1 && !is_f32<R>() && !XD;
@@ -671,7 +671,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(V == 1 ? 
       int bflags = 0;
       int e;
       if constexpr (HOT) {
-         const HotPlan<R>* h = &hot;
+         const HotPlan* h = &hot;
          e = gc_step<R, BG, XD, V>(h, Pi, Li, rng, first, slot, H, C, tid, bflags);
       }
       else e = gc_step<R, BG, XD, V>(Pi, Pi, Li, rng, first, slot, H, C, tid, bflags);

@@ -45,7 +45,7 @@ struct Launch {
    const QueryDesc* queries;            // query table
    const int32_t* queue;                // admitted query indices, oldest first
    int32_t n_queue;
-   int32_t steps_per_launch;
+   int32_t n_queries;                   // size of the query table
    uint64_t n_lanes;                    // a multiple of the block size: waves are always full
    int32_t* slot_q;                     // query index of each slot (-1: none)
    // lane state (structure of arrays, n_lanes each; boundary arrays SPX_MAX_BND * n_lanes)
@@ -75,7 +75,6 @@ struct Launch {
    int32_t* rank;
    uint32_t* n_running;
    int32_t* list;
-   int32_t n_queries, pad_;             // size of the query table
 };
 
 // Slot states

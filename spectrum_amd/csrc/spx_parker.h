@@ -1,11 +1,12 @@
 // spx_parker.h -- Parker and Parker-with-source transport kernels for gfx950 (MI355X).
 //
-// One lane per trajectory slot; the slots of a run are resident in HBM as structure-of-arrays state.
-// Each engine launch is a pair of kernels, both captured together in a HIP graph for steady loops:
+// One lane per trajectory slot, or four in the step kernels for few waves; the slots of a run are resident in HBM as
+// structure-of-arrays state.  Each engine launch is a pair of kernels, with a packing pass between them where the
+// running slots are packed into full waves, and both are captured together in a HIP graph for steady loops:
 //   * the service kernel refills idle slots from the device work counter (one atomic per wave),
 //     runs SetStart, bins pending distribution events, retries discarded attempts and writes the
 //     per-trajectory records;
-//   * the step kernel advances every running slot by up to `steps_per_launch` steps with the hot
+//   * the step kernel advances every running slot by up to LaunchShape::n_steps steps with the hot
 //     state in registers; a slot that produces a distribution event or ends stops there and waits
 //     for the next service pass.
 // The step reproduces TrajectoryParker::Advance (src/trajectory_parker.cc:255-306) with the Euler
@@ -710,7 +711,7 @@ __device__ __forceinline__ void parker_step_body(const Launch* __restrict__ Lg, 
    int st = run ? SLOT_RUN : SLOT_IDLE;
    int exc = 0;
    unsigned long long steps_here = 0;
-   HotPlan<R> hot;
+   HotPlan hot;
    // the gridded step's plan is too large to keep (420 registers, most of them spilled: 10% slower than reading it)
    constexpr bool HOT = V == 1 && !is_f32<R>() && BG != SPX_BG_GRID;
    if constexpr (HOT) load_hot(hot, P);
@@ -732,7 +733,7 @@ __device__ __forceinline__ void parker_step_body(const Launch* __restrict__ Lg, 
       // 1.67 -> 1.86e10 steps/s, 25^3 2.12 -> 2.46e10, anisotropic kappa 3.10 -> 3.17e9 and 3.97 -> 4.01e9.
       if constexpr (BG == SPX_BG_GRID && V == 0 && is_f32<R>()) asm volatile("" : "+v"(H.rs.traj));
       if constexpr (HOT) {
-         const HotPlan<R>* h = &hot;
+         const HotPlan* h = &hot;
          e = (TT == 2) ? fieldline_step<R, BG, FWD, V>(h, Pi, Li, slot, H, C, tid, bflags)
                        : parker_step<R, BG, FWD, TT, DF, V>(h, Pi, Li, rng, first, slot, H, C, tid, bflags);
       }

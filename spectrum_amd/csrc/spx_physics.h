@@ -179,13 +179,12 @@ typedef const SPX_CP spx_plan_desc* PlanPtr;
 // resident waves hide; with one wave per SIMD nothing does (2.4 of 20.3 thousand cycles of that step).  The FP32
 // kernels always read the plan: from a copy the optimizer takes reciprocals of its members out of the loop and lays
 // out other basic blocks, and with contraction across statements the step then rounds differently.
-template <typename R>
 struct HotPlan {
    int32_t traj_type, n_bnd, n_bt;
    int64_t max_steps;
    double dt_scale, src_p_inj, src_rate;
-   spx_bg_t<R> vbg;
-   spx_df_t<R> vdf;
+   spx_bg_t<double> vbg;
+   spx_df_t<double> vdf;
    spx_bnd_desc bnd[SPX_MAX_BND];
 };
 
@@ -194,25 +193,18 @@ template <typename R> struct PlanView;
 template <> struct PlanView<double> {
    static __device__ const SPX_CP spx_bg_t<double>& bg(PlanPtr P) { return P->bg; }
    static __device__ const SPX_CP spx_df_t<double>& df(PlanPtr P) { return P->df; }
-   static __device__ const spx_bg_t<double>& bg(const HotPlan<double>* P) { return P->vbg; }
-   static __device__ const spx_df_t<double>& df(const HotPlan<double>* P) { return P->vdf; }
+   static __device__ const spx_bg_t<double>& bg(const HotPlan* P) { return P->vbg; }
+   static __device__ const spx_df_t<double>& df(const HotPlan* P) { return P->vdf; }
 };
 template <> struct PlanView<float> {
    static __device__ const SPX_CP spx_bg_t<float>& bg(PlanPtr P) { return P->bgf; }
    static __device__ const SPX_CP spx_df_t<float>& df(PlanPtr P) { return P->dff; }
-   static __device__ const spx_bg_t<float>& bg(const HotPlan<float>* P) { return P->vbg; }
-   static __device__ const spx_df_t<float>& df(const HotPlan<float>* P) { return P->vdf; }
 };
 
-__device__ __forceinline__ const spx_bg_t<double>& hot_bg(const spx_plan_desc* g, double*) { return g->bg; }
-__device__ __forceinline__ const spx_bg_t<float>& hot_bg(const spx_plan_desc* g, float*) { return g->bgf; }
-__device__ __forceinline__ const spx_df_t<double>& hot_df(const spx_plan_desc* g, double*) { return g->df; }
-__device__ __forceinline__ const spx_df_t<float>& hot_df(const spx_plan_desc* g, float*) { return g->dff; }
 // Each member goes through an empty asm: its value is then opaque, so the register allocator cannot repeat the
 // load inside the step loop in place of keeping it.  Members that nothing reads disappear.  Numbers go to vector
 // registers (free where few waves are resident), what branches read to scalar ones.
 __device__ __forceinline__ void opaque(double& d) { asm("" : "+v"(d)); }
-__device__ __forceinline__ void opaque(float& d) { asm("" : "+v"(d)); }
 __device__ __forceinline__ void opaque(int32_t& d) { asm("" : "+s"(d)); }
 __device__ __forceinline__ void opaque(int64_t& d) { asm("" : "+s"(d)); }
 template <typename T> __device__ __forceinline__ void opaque(const T*& d) { asm("" : "+s"(d)); }
@@ -224,15 +216,14 @@ struct HotLoad {
       for (int i = 0; i < N; i++) (*this)(d[i], s[i]);
    }
 };
-template <typename R>
-__device__ __forceinline__ void load_hot(HotPlan<R>& h, PlanPtr P)
+__device__ __forceinline__ void load_hot(HotPlan& h, PlanPtr P)
 {
    const HotLoad keep;
    const spx_plan_desc* g = (const spx_plan_desc*)P;   // the compiler follows the address space through the cast
 #define SPX_HOT(m) keep(h.m, g->m)
    SPX_HOT(traj_type); SPX_HOT(n_bnd); SPX_HOT(n_bt); SPX_HOT(max_steps); SPX_HOT(dt_scale); SPX_HOT(src_p_inj); SPX_HOT(src_rate);
 #undef SPX_HOT
-   const spx_bg_t<R>& b = hot_bg(g, (R*)nullptr);
+   const spx_bg_t<double>& b = g->bg;
 #define SPX_HOT(m) keep(h.vbg.m, b.m)
    SPX_HOT(kind); SPX_HOT(ep_diag); SPX_HOT(t0); SPX_HOT(r0); SPX_HOT(u0); SPX_HOT(B0); SPX_HOT(dmax0); SPX_HOT(r_ref); SPX_HOT(dmax_fraction);
    SPX_HOT(eprime[0]); SPX_HOT(eprime[1]); SPX_HOT(eprime[2]); SPX_HOT(ur0); SPX_HOT(w0); SPX_HOT(hp_rad); SPX_HOT(ur0_rcp); SPX_HOT(sw_c1);
@@ -242,7 +233,7 @@ __device__ __forceinline__ void load_hot(HotPlan<R>& h, PlanPtr P)
    SPX_HOT(grid.f_vel); SPX_HOT(grid.f_mag); SPX_HOT(grid.bmag_min); SPX_HOT(grid.inner_lo); SPX_HOT(grid.inner_hi); SPX_HOT(grid.fd_fields);
    SPX_HOT(grid.z64); SPX_HOT(grid.c32);
 #undef SPX_HOT
-   const spx_df_t<R>& f = hot_df(g, (R*)nullptr);
+   const spx_df_t<double>& f = g->df;
 #define SPX_HOT(m) keep(h.vdf.m, f.m)
    SPX_HOT(kind); SPX_HOT(stream_dep_idx); SPX_HOT(pos_dep); SPX_HOT(iso_r); SPX_HOT(region_idx); SPX_HOT(D0); SPX_HOT(Dperp); SPX_HOT(Dpara); SPX_HOT(kap0);
    SPX_HOT(U0); SPX_HOT(pow_law_U); SPX_HOT(p0); SPX_HOT(pow_law_p); SPX_HOT(kap_rat); SPX_HOT(T0); SPX_HOT(r0); SPX_HOT(pow_law_T);

@@ -178,7 +178,6 @@ hipError_t Pool::init(const spx_plan_desc& s, int prec, uint64_t lanes, int spl,
    host.queries = queries.p;
    host.queue = queue.p;
    host.n_queue = 0;
-   host.steps_per_launch = spl;
    host.n_lanes = n;
    host.slot_q = slot_q.p;
    host.active = active.p;

@@ -159,7 +159,6 @@ hipError_t static_run(const spx_plan_desc& plan, int precision, int steps_per_la
       comps += (int64_t)plan.dist[d].nb * plan.dist[d].width;
    }
    if (bins > SPX_STATIC_BINS || comps > SPX_STATIC_COMPONENTS) return hipErrorInvalidValue;
-   R.host.steps_per_launch = steps_per_launch;
 
    QueryDesc q;
    std::memset(&q, 0, sizeof(q));
