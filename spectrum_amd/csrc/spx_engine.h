@@ -829,7 +829,6 @@ __device__ __forceinline__ void service_slot(LaunchPtr L, int32_t packed, StartF
          }
       }
    }
-   L->slot_q[slot] = q;
    // 4. SetStart, repeated with continuing draws when an attempt is discarded
    if (st == SLOT_START) {
       const QueryPtr Q = query_of(L, q);
@@ -860,7 +859,7 @@ __device__ __forceinline__ void service_slot(LaunchPtr L, int32_t packed, StartF
    }
    L->active[slot] = st;
    // a wave whose last trajectories have failed in SetStart leaves its query now: once complete, the query's memory goes
-   if (__ballot(st != SLOT_IDLE) == 0) L->slot_q[slot] = -1;
+   L->slot_q[slot] = __ballot(st != SLOT_IDLE) == 0 ? -1 : q;
    // 5. for a packed launch: this slot's place among the running slots of its query (one atomic per wave)
    if (packed >= 0) {
       const uint64_t mask = __ballot(st == SLOT_RUN);
