@@ -433,7 +433,7 @@ __device__ int gc_set_start(PlanPtr P, QueryPtr Q, LaunchPtr L, const spx_rng_de
 }
 
 template <typename R, int BG>
-__global__ __launch_bounds__(BLOCK) void gc_service(const Launch* __restrict__ Lg, int32_t packed)
+__global__ __launch_bounds__(SERVICE_BLOCK) void gc_service(const Launch* __restrict__ Lg, int32_t packed)
 {
    const LaunchPtr L = (LaunchPtr)Lg;
    service_slot(L, packed, [&](PlanPtr P, QueryPtr Q, const spx_rng_desc& rng, uint64_t slot, uint64_t traj, uint32_t& nu) {
@@ -710,7 +710,7 @@ template <typename R, int BG, bool XD, int M>
 static hipError_t launch_gc_bg(const LaunchShape& S, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
 {
    if constexpr (M != LAUNCH_FEW) {
-      hipLaunchKernelGGL((gc_service<R, BG>), dim3(service_grid(S)), dim3(BLOCK), 0, st, d_launch, S.packed);
+      hipLaunchKernelGGL((gc_service<R, BG>), dim3(service_grid(S)), dim3(SERVICE_BLOCK), 0, st, d_launch, S.packed);
       if (S.packed >= 0) {
          hipError_t e = pack_running(S, d_launch, st);
          if (e != hipSuccess) return e;

@@ -118,7 +118,7 @@ __device__ int lz_set_start(PlanPtr P, QueryPtr Q, LaunchPtr L, const spx_rng_de
 }
 
 template <typename R, int BG>
-__global__ __launch_bounds__(BLOCK) void lz_service(const Launch* __restrict__ Lg, int32_t packed)
+__global__ __launch_bounds__(SERVICE_BLOCK) void lz_service(const Launch* __restrict__ Lg, int32_t packed)
 {
    const LaunchPtr L = (LaunchPtr)Lg;
    service_slot(L, packed, [&](PlanPtr P, QueryPtr Q, const spx_rng_desc& rng, uint64_t slot, uint64_t traj, uint32_t& nu) {
@@ -256,7 +256,7 @@ __global__ __launch_bounds__(BLOCK) void lz_step_kernel(const Launch* __restrict
 template <typename R, int BG, int FWD>
 static hipError_t launch_lz_bg(const LaunchShape& S, const Launch* d_launch, hipStream_t st, hipEvent_t mid)
 {
-   hipLaunchKernelGGL((lz_service<R, BG>), dim3(service_grid(S)), dim3(BLOCK), 0, st, d_launch, S.packed);
+   hipLaunchKernelGGL((lz_service<R, BG>), dim3(service_grid(S)), dim3(SERVICE_BLOCK), 0, st, d_launch, S.packed);
    if (S.packed >= 0) {
       hipError_t e = pack_running(S, d_launch, st);
       if (e != hipSuccess) return e;
