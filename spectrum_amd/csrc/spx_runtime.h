@@ -131,6 +131,7 @@ private:
    double ms_per_step = 0.0;            // of the last round, and what it was asked to last
    double round_ms = 0.0;
    uint64_t round_live = 0;
+   int round_n = 0;                     // launches of the last round
 };
 
 }  // namespace spx
